@@ -375,6 +375,9 @@ class Model(nn.Module):
             return steps
 
         if entry is None:
+            # Fuse before the capture: a fusion inside it would be recorded and not run, and every replay would
+            # read the separate weights, which fusing frees.
+            self._fused_projections()
             buffers = [(torch.empty(2, b - a, dtype=torch.int64, device=cache.device),
                         torch.empty(b - a, dtype=torch.int64, device=cache.device)) for a, b in spans]
             steps = open_steps(buffers)

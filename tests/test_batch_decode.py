@@ -327,3 +327,30 @@ def test_graph_replayed_decode_equals_the_eager_decode(gpu, micro_batches):
     assert "_decode_graphs" not in model.__dict__
     fresh.step()  # captures again
     assert len(model.__dict__["_decode_graphs"]) == 1
+
+
+@pytest.mark.gpu
+def test_first_graph_step_fuses_the_projections_outside_the_capture(gpu, monkeypatch):
+    """A model whose first batched step is a graph step fuses its projections
+    before the capture: fused inside it, the concatenation would be recorded
+    instead of run and each replay would read the freed separate weights."""
+    from nano_hisparse import model as model_module
+
+    log_case(test="fuse-before-capture")
+    cfg = ModelConfig(vocab_size=64, hidden_size=2048, intermediate_size=2048, num_hidden_layers=2,
+                      num_attention_heads=16, num_key_value_heads=4)
+    torch.manual_seed(5)
+    model = Model(cfg).eval().to(gpu, torch.bfloat16)
+    fuse, capturing = model_module._fuse, []
+
+    def recording(*a):
+        capturing.append(torch.cuda.is_current_stream_capturing())
+        return fuse(*a)
+
+    monkeypatch.setattr(model_module, "_fuse", recording)
+    kv = CacheConfig(gpu_pages=64, host_pages=64, page_size=4, kv_heads=4, head_dim=128, dtype=torch.bfloat16,
+                     device=str(gpu))
+    engine = Engine(model, HybridKVCache(kv, HotConfig(16, 16)), top_k=4, batch_decode=True, graph=True)
+    engine.add_request("r", list(range(1, 20)), 4)
+    engine.run()
+    assert capturing and not any(capturing)
