@@ -667,3 +667,15 @@ def test_append_page_matches_oracle(gpu, dtype, P, Hkv, D):
         assert torch.equal(lo.float().cpu(), e_lo) and torch.equal(hi.float().cpu(), e_hi)
     others = [i for i in range(host_pages) if i != host_page]
     assert torch.equal(host[others].view(torch.uint8), host_before[others].view(torch.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,P,Hkv,D", [
+    (torch.bfloat16, 100, 2, 40),  # more rows than one pass holds, a partial last group of chunks
+    (torch.float16, 130, 3, 8),  # three passes, three chunks
+    (torch.float32, 65, 1, 20), (torch.float32, 32, 8, 128),  # 4-byte elements: 4 per chunk
+    (torch.bfloat16, 64, 1, 8),  # one chunk
+    (torch.bfloat16, 40, 1, 12),  # rows that are no whole chunks (one thread per element)
+])
+def test_append_rows_at_the_edges_of_passes_and_chunks(gpu, dtype, P, Hkv, D):
+    test_append_page_matches_oracle(gpu, dtype, P, Hkv, D)
