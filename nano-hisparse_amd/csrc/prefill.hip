@@ -2,51 +2,68 @@
 //
 // out[s, h] = softmax_{t <= s}(q[s, h] . k[t, h/g] * D^-1/2) . v[t, h/g] for
 // one prompt of `seq` tokens, bf16 or fp16 in, fp32 accumulation. A
-// workgroup of 8 waves owns 128 queries of one query head (16 per wave) and
-// walks the key tiles of 64 up to the diagonal with an online softmax.
+// workgroup of NW waves owns 32 * NW queries of one query head (32 per wave)
+// and walks the key tiles of 64 up to the diagonal with an online softmax.
 //
-// MFMA v_mfma_f32_16x16x32 (bf16 / f16): lane l supplies row l%16 of A and
-// column l%16 of B at k = (l/16)*8 .. +7, and receives D rows (l/16)*4 + i,
-// column l%16. The scores are computed transposed, S^T = K Q^T (A = 16 key
-// rows of the LDS K tile, B = the wave's 16 query rows kept in registers),
-// so a lane holds keys (l/16)*4 + i of every 16-key block for its query
-// column l%16: a query's softmax statistics live in the 4 lanes l%16 = n and
-// are reduced with two lane swaps. The output is accumulated transposed too,
-// O^T = V^T P^T: its B operand (P^T, keys x queries) is the score layout
-// itself once the k index of a 32-key step is taken as (block 2j, keys
-// (l/16)*4 + i) then (block 2j+1, keys (l/16)*4 + i) -- the A operand (V^T
-// rows from the transposed LDS V tile) uses the same key order -- and the
-// rescaling by a query's max stays in its lane. The weights are rounded to
-// the input dtype for the P.V product and the denominator sums the same
-// rounded weights, so each output is an exact convex combination of V rows.
+// MFMA v_mfma_f32_32x32x16 (bf16 / f16): lane l supplies row l%32 of A and
+// column l%32 of B at k = (l/32)*8 .. +7, and receives D rows
+// 8*(i/4) + (l/32)*4 + i%4 (i = 0..15) of column l%32. The scores are
+// computed transposed, S^T = K Q^T (A = 32 key rows of the LDS K tile, B =
+// the wave's 32 query rows, kept in registers), so a lane holds 16 keys of
+// every 32-key block for its query column l%32 and a query's softmax
+// statistics live in the lane pair l, l ^ 32. The output is accumulated
+// transposed too, O^T = V^T P^T: registers 8s .. 8s+7 of a score block are
+// the B operand of k step s as they stand once the step's 16 keys are taken
+// in the order (l/32)*4 + 0..3, 8 + (l/32)*4 + 0..3, and the LDS V^T tile
+// stores each 16 keys in that order, so its A operand is one 16-byte read.
+// The rescaling by a query's max stays in its lane.
+//
+// Why 32 queries per wave and 32x32 tiles: a wave reads every K and V byte
+// of the tile from LDS once per MFMA operand, so the LDS bytes per flop fall
+// with the queries a wave holds. At 16 per wave (16x16 tiles) the LDS reads
+// took twice the matrix cores' time; at 32 they take as long as it does, and
+// the wave still fits 256 registers, so two waves share a SIMD and one's
+// softmax runs beside the other's MFMAs. K and V^T rows are stored with their
+// 16-byte chunks permuted by an XOR of the row, so that reads of 16 rows at
+// one chunk meet all 64 banks.
+//
+// The weights are rounded to the input dtype for the P.V product and the
+// denominator sums the same rounded weights, so each output is an exact
+// convex combination of V rows. A tile that moves no query's max rescales
+// nothing. (Moving the max only once a score exceeds it by 2^8 would skip
+// more, 3% of the time at 32K tokens, but the largest weight would no longer
+// be exactly 1: the error against float64 grew by 3%.)
+//
+// Measured (MI355X, bf16, 32/8 heads of 128): 32768 tokens 8.86 ms, 993
+// TFLOP/s causal (22.37 ms with 16 queries per wave and 16x16 tiles; a large
+// hipBLASLt product reaches 1342); 4000 tokens 157 us (605); 1999 tokens of
+// 28/4 heads 63 us (159), where the longest workgroup's 32 tiles of ~2 us
+// are the bound and the chip is half idle.
 #include <math.h>
 
 #include "nhs_common.h"
 
 namespace nhs {
 
-constexpr int kPfWaves = 8;
-constexpr int kPfThreads = kPfWaves * kWave;
-constexpr int kPfBM = 16 * kPfWaves;  // queries per workgroup
-constexpr int kPfBN = 64;             // keys per tile
+constexpr int kPfBN = 64;            // keys per tile
+constexpr int kPfCUs = 256;
 
 typedef __bf16 pf_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_f16x8 __attribute__((ext_vector_type(8)));
-typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ __forceinline__ pf_f32x4 mfma16x16x32(uint4 a, uint4 b, pf_f32x4 c) {
-  if constexpr (T::dtype == NHS_BF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, a), __builtin_bit_cast(pf_bf16x8, b),
-                                                  c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pf_f16x8, a), __builtin_bit_cast(pf_f16x8, b), c,
-                                                 0, 0, 0);
-}
-
+typedef float pf_f32x16 __attribute__((ext_vector_type(16)));
 typedef float pf_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 pf_bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 pf_f16x2 __attribute__((ext_vector_type(2)));
+
+template <typename T>
+__device__ __forceinline__ pf_f32x16 mfma32x32x16(uint4 a, uint4 b, pf_f32x16 c) {
+  if constexpr (T::dtype == NHS_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pf_bf16x8, a), __builtin_bit_cast(pf_bf16x8, b),
+                                                  c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_f16x8, a), __builtin_bit_cast(pf_f16x8, b), c,
+                                                 0, 0, 0);
+}
 
 // two fp32 weights as a packed pair of the input dtype (round to nearest
 // even, by the hardware conversions)
@@ -57,16 +74,20 @@ __device__ __forceinline__ uint32_t pf_pack(float lo, float hi) {
   else
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((pf_f32x2){lo, hi}, pf_f16x2));
 }
+
+// acc + both halves of a packed pair, in fp32
 template <typename T>
-__device__ __forceinline__ float pf_unpack(uint32_t v, int half) {
-  const uint32_t b = half ? v >> 16 : v & 0xffffu;
-  return T::dtype == NHS_BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b);
+__device__ __forceinline__ float pf_add_pair(uint32_t pair, float acc) {
+  if constexpr (T::dtype == NHS_BF16)
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pf_bf16x2, pair),
+                                           __builtin_bit_cast(pf_bf16x2, 0x3f803f80u), acc, false);
+  else
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(pf_f16x2, pair), __builtin_bit_cast(pf_f16x2, 0x3c003c00u), acc,
+                                  false);
 }
 
-// 16-bit element (word w, half) of a 16-byte chunk
-__device__ __forceinline__ uint32_t pf_get16(const uint4& v, int w, int half) {
-  const uint32_t x = w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w;
-  return half ? x >> 16 : x & 0xffffu;
+__device__ __forceinline__ uint32_t pf_word(const uint4& v, int w) {
+  return w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w;
 }
 
 struct PrefillArgs {
@@ -80,84 +101,113 @@ struct PrefillArgs {
   int64_t o_s, o_h;
 };
 
-template <typename T, int D>
-__global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillArgs a) {
-  constexpr int KS = D / 32;   // 32-wide k steps of Q.K
-  constexpr int DB = D / 16;   // 16-wide dim blocks of the output
-  constexpr int KROW = D * 2 + 16;       // bytes per K row in LDS (padded)
-  constexpr int VROW = kPfBN * 2 + 16;   // bytes per V^T row in LDS (padded)
+// LDS slot of 16-byte chunk c of K row r (D * 2 bytes) and of V^T row r (128 bytes): any 16 consecutive rows at one
+// chunk fall on distinct banks.
+template <int D>
+__device__ __forceinline__ int pf_k_slot(int r, int c) {
+  return D == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7);
+}
+__device__ __forceinline__ int pf_v_slot(int r, int c) { return c ^ (((r >> 1) ^ (r >> 4)) & 7); }
+
+template <typename T, int D, int NW>
+__global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(PrefillArgs a) {
+  constexpr int kThreads = NW * kWave;
+  constexpr int BM = 32 * NW;          // queries per workgroup
+  constexpr int KS = D / 16;           // 16-wide k steps of Q.K
+  constexpr int DB = D / 32;           // 32-wide dim blocks of the output
+  constexpr int C = D / 8;             // 16-byte chunks of a K or V row
+  constexpr int kVRow = kPfBN * 2;     // bytes per V^T row
+  // a staging unit is four 16-byte loads: 4 keys x 8 dims of V (a 4-key piece of 8 V^T rows), or one chunk of 4 K rows
+  constexpr int kUnits = kPfBN * D / 32;  // units per tile of each
+  constexpr int kMine = (2 * kUnits + kThreads - 1) / kThreads;
   // two buffers per tile: tile t+1 is stored while tile t is read, one barrier per tile
-  __shared__ __attribute__((aligned(16))) char ks_buf[2][kPfBN * KROW];
-  __shared__ __attribute__((aligned(16))) char vt_buf[2][D * VROW];
+  __shared__ __attribute__((aligned(16))) char k_buf[2][kPfBN * D * 2];
+  __shared__ __attribute__((aligned(16))) char v_buf[2][D * kVRow];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g4 = lane >> 4, n = lane & 15;
-  const int n_qblocks = (a.seq + kPfBM - 1) / kPfBM;
-  const int qb = n_qblocks - 1 - (int)blockIdx.x;  // the longest rows first
-  const int h = blockIdx.y;
+  const int half = lane >> 5, n = lane & 31;
+  // The longest rows first; with a multiple of 8 heads each XCD (workgroup id mod 8) keeps neighbouring heads, so that
+  // the heads of one KV head read its tiles from one L2.
+  const int n_qblocks = (a.seq + BM - 1) / BM;
+  const int id = blockIdx.x;
+  const int h = a.q_heads % 8 == 0 ? (id % 8) * (a.q_heads / 8) + (id / 8) % (a.q_heads / 8) : id % a.q_heads;
+  const int qb = n_qblocks - 1 - id / a.q_heads;
   const int kvh = h / a.group;
-  const int q0 = qb * kPfBM;
-  const int query = q0 + wave * 16 + n;  // this lane's query (column of S^T)
-  const bool q_live = query < a.seq;
+  const int q0 = qb * BM, wq0 = q0 + wave * 32;
+  const int query = wq0 + n;  // this lane's query (column of S^T)
 
-  // the wave's query rows as B operands: dims ks*32 + g4*8 .. +7
+  // the wave's query rows as B operands: dims s*16 + half*8 .. +7
   uint4 qf[KS];
   {
-    const int qr = q_live ? query : a.seq - 1;
-    const char* qp = a.q + ((int64_t)qr * a.q_s + (int64_t)h * a.q_h) * T::bytes;
+    const int qr = min(query, a.seq - 1);
+    const char* qp = a.q + ((int64_t)qr * a.q_s + (int64_t)h * a.q_h) * T::bytes + half * 16;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uint4*>(qp + (s * 32 + g4 * 8) * T::bytes);
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uint4*>(qp + s * 32);
   }
 
-  float m = -INFINITY, l = 0.f;
-  pf_f32x4 o[DB];
+  float m = -INFINITY, l = 0.f;  // running max (of the unscaled scores) and this lane's share of the denominator
+  pf_f32x16 o[DB];
 #pragma unroll
-  for (int b = 0; b < DB; ++b) o[b] = (pf_f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[b][i] = 0.f;
 
-  // tile staging: thread t loads K row t/KT's dims [(t%KT)*D/KT, +D/KT) and
-  // the VR V rows VR*(t/16) .. +VR-1 at dims 8*(t%16) .. +7 (D = 64 uses the
-  // first half of the threads for V)
-  constexpr int KT = kPfThreads / kPfBN;        // threads per K row
-  constexpr int KCH = D * 2 / KT / 16;          // 16-byte chunks of K per thread
-  constexpr int VR = kPfBN * 16 / kPfThreads;   // V rows per thread (16 groups of 8 dims)
-  static_assert(KCH >= 1 && (VR == 2 || VR == 4), "tile staging layout");
-  const int krow = tid / KT, kcol = (tid % KT) * (D / KT);
-  const int vkg = tid >> 4, vdg = tid & 15;
-  const bool v_thread = vdg * 8 < D;
-  const int last_key = min(a.seq, q0 + kPfBM) - 1;
+  const int last_key = min(a.seq, q0 + BM) - 1;
   const int n_tiles = last_key / kPfBN + 1;
-  uint4 kreg[KCH], vreg[VR];
+  const char* kbase = a.k + (int64_t)kvh * a.k_h * T::bytes;
+  const char* vbase = a.v + (int64_t)kvh * a.v_h * T::bytes;
+  uint4 reg[kMine][4];
   auto load_tile = [&](int t0) {
-    const int kr = min(t0 + krow, a.seq - 1);  // rows past the end re-read the last key (masked below)
-    const char* kp = a.k + ((int64_t)kr * a.k_s + (int64_t)kvh * a.k_h + kcol) * T::bytes;
 #pragma unroll
-    for (int c = 0; c < KCH; ++c) kreg[c] = *reinterpret_cast<const uint4*>(kp + c * 16);
-    if (v_thread)
+    for (int u = 0; u < kMine; ++u) {
+      const int unit = tid + u * kThreads;
+      const bool is_v = unit < kUnits;
+      if (unit >= 2 * kUnits) break;
+      const int x = is_v ? unit : unit - kUnits;
+      const int row = is_v ? (x / C) * 4 : x / C, step = is_v ? 1 : kPfBN / 4;
+      const char* base = (is_v ? vbase : kbase) + (x % C) * 16;
+      const int64_t stride = (is_v ? a.v_s : a.k_s) * T::bytes;
+      if (t0 + kPfBN <= a.seq) {
+        const char* p = base + (int64_t)(t0 + row) * stride;
 #pragma unroll
-      for (int r = 0; r < VR; ++r) {
-        const int vr = min(t0 + vkg * VR + r, a.seq - 1);
-        vreg[r] = *reinterpret_cast<const uint4*>(a.v + ((int64_t)vr * a.v_s + (int64_t)kvh * a.v_h + vdg * 8) * T::bytes);
+        for (int i = 0; i < 4; ++i) reg[u][i] = *reinterpret_cast<const uint4*>(p + i * step * stride);
+      } else {  // rows past the end re-read the last key (masked below)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          reg[u][i] = *reinterpret_cast<const uint4*>(base + (int64_t)min(t0 + row + i * step, a.seq - 1) * stride);
       }
+    }
   };
   auto store_tile = [&](int buf) {
-    char* ks_lds = ks_buf[buf];
-    char* vt_lds = vt_buf[buf];
 #pragma unroll
-    for (int c = 0; c < KCH; ++c)
-      *reinterpret_cast<uint4*>(ks_lds + krow * KROW + kcol * T::bytes + c * 16) = kreg[c];
-    if (v_thread)
+    for (int u = 0; u < kMine; ++u) {
+      const int unit = tid + u * kThreads;
+      if (unit >= 2 * kUnits) break;
+      if (unit < kUnits) {
+        const int kg = unit / C, r0 = (unit % C) * 8;  // keys 4 kg .. +3, dims r0 .. +7
+        const int c = 2 * (kg >> 2) + (kg & 1), piece = (kg >> 1) & 1;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {  // V^T[dim 8*vdg + j][keys VR*vkg .. +VR-1]
-        const int half = j & 1, w = j >> 1;
-        const uint32_t e0 = pf_get16(vreg[0], w, half), e1 = pf_get16(vreg[1], w, half);
-        char* dst = vt_lds + (vdg * 8 + j) * VROW + vkg * VR * 2;
-        if constexpr (VR == 4) {
-          const uint32_t e2 = pf_get16(vreg[2], w, half), e3 = pf_get16(vreg[3], w, half);
-          *reinterpret_cast<uint2*>(dst) = make_uint2(e0 | (e1 << 16), e2 | (e3 << 16));
-        } else {
-          *reinterpret_cast<uint32_t*>(dst) = e0 | (e1 << 16);
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+          const uint32_t lo = __builtin_amdgcn_perm(pf_word(reg[u][1], j >> 1), pf_word(reg[u][0], j >> 1), sel);
+          const uint32_t hi = __builtin_amdgcn_perm(pf_word(reg[u][3], j >> 1), pf_word(reg[u][2], j >> 1), sel);
+          *reinterpret_cast<uint2*>(v_buf[buf] + (r0 + j) * kVRow + pf_v_slot(r0 + j, c) * 16 + piece * 8) =
+              make_uint2(lo, hi);
+        }
+      } else {
+        const int x = unit - kUnits, c = x % C;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = x / C + i * (kPfBN / 4);
+          *reinterpret_cast<uint4*>(k_buf[buf] + r * (D * 2) + pf_k_slot<D>(r, c) * 16) = reg[u][i];
         }
       }
+    }
+  };
+
+  auto stage = [&](int t) {
+    store_tile((t + 1) & 1);
+    if (t + 2 < n_tiles) load_tile((t + 2) * kPfBN);  // in flight during the rest of tile t's math and tile t+1's QK
   };
 
   load_tile(0);
@@ -166,94 +216,117 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillAr
   for (int t = 0; t < n_tiles; ++t) {
     const int t0 = t * kPfBN;
     // tile t's buffer is complete and every wave is done with tile t-1's
-    // buffer, which now takes tile t+1 (loaded during tile t-1's math)
+    // buffer, which takes tile t+1 (loaded during tile t-1's math)
     __syncthreads();
-    if (t + 1 < n_tiles) {
-      store_tile((t + 1) & 1);
-      if (t + 2 < n_tiles) load_tile(t0 + 2 * kPfBN);  // in flight during this tile's math
+    // the next tile is stored under the first MFMAs (waves without queries in this tile store it alone)
+    const bool stages = t + 1 < n_tiles;
+    if (t0 > wq0 + 31) {  // wholly above the wave's diagonal
+      if (stages) stage(t);
+      continue;
     }
-    const char* ks_lds = ks_buf[t & 1];
-    const char* vt_lds = vt_buf[t & 1];
+    const char* kl = k_buf[t & 1] + n * (D * 2);
+    const char* vl = v_buf[t & 1] + n * kVRow;
 
-    // S^T for 4 key blocks of 16: s[kb] holds keys t0 + kb*16 + g4*4 + i
-    pf_f32x4 s[4];
+    // S^T for 2 key blocks of 32: s[kb][i] holds key t0 + kb*32 + (i/4)*8 + half*4 + i%4
+    pf_f32x16 s[2];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      s[kb] = (pf_f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int st = 0; st < KS; ++st) {
-        const uint4 kf = *reinterpret_cast<const uint4*>(ks_lds + (kb * 16 + n) * KROW + (st * 32 + g4 * 8) * T::bytes);
-        s[kb] = mfma16x16x32<T>(kf, qf[st], s[kb]);
+      for (int i = 0; i < 16; ++i) s[kb][i] = 0.f;
+#pragma unroll
+    for (int st = 0; st < KS; ++st)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const uint4 kf =
+            *reinterpret_cast<const uint4*>(kl + kb * 32 * D * 2 + pf_k_slot<D>(n, 2 * st + half) * 16);
+        s[kb] = mfma32x32x16<T>(kf, qf[st], s[kb]);
       }
-    }
-    // scale, mask (causal and past the end; a tile wholly below the wave's
-    // diagonal and inside the prompt needs none), running max
-    float mx = m;
-    if (t0 + kPfBN - 1 <= q0 + wave * 16 && t0 + kPfBN <= a.seq) {  // uniform over the wave
+    if (stages) stage(t);
+    // causal and past-the-end mask (a tile wholly below the wave's diagonal
+    // and inside the prompt needs none)
+    if (t0 + kPfBN - 1 > wq0 || t0 + kPfBN > a.seq) {  // uniform over the wave
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          s[kb][i] = s[kb][i] * a.scale_log2;
-          mx = fmaxf(mx, s[kb][i]);
-        }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = t0 + kb * 16 + g4 * 4 + i;
-          const float x = (key <= query && key < a.seq) ? s[kb][i] * a.scale_log2 : -INFINITY;
-          s[kb][i] = x;
-          mx = fmaxf(mx, x);
+        for (int i = 0; i < 16; ++i) {
+          const int key = t0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+          if (key > query || key >= a.seq) s[kb][i] = -INFINITY;
         }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kb][i]);
     mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float ref = mx == -INFINITY ? 0.f : mx;
-    const float alpha = __builtin_amdgcn_exp2f(m - ref);
-    m = mx;
-    // weights rounded to the input dtype, packed as P^T B operands: step j
-    // (keys of blocks 2j and 2j+1) is {s[2j][0..3], s[2j+1][0..3]}
-    uint4 pb[2];
-    float psum = 0.f;
+    if (__any(mx > m)) {
+      const float moved = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f((m - (moved == -INFINITY ? 0.f : moved)) * a.scale_log2);
+      m = moved;
+      l *= alpha;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][i] *= alpha;
+    }
+    const float ref = m == -INFINITY ? 0.f : m * a.scale_log2;
+    // weights rounded to the input dtype, packed as P^T B operands
+    uint4 pb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
       uint32_t w[4];
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const pf_f32x4& sv = s[2 * j + half];
-        const uint32_t a01 = pf_pack<T>(__builtin_amdgcn_exp2f(sv[0] - ref), __builtin_amdgcn_exp2f(sv[1] - ref));
-        const uint32_t a23 = pf_pack<T>(__builtin_amdgcn_exp2f(sv[2] - ref), __builtin_amdgcn_exp2f(sv[3] - ref));
-        w[half * 2] = a01, w[half * 2 + 1] = a23;
-        psum += pf_unpack<T>(a01, 0) + pf_unpack<T>(a01, 1) + pf_unpack<T>(a23, 0) + pf_unpack<T>(a23, 1);
+      for (int x = 0; x < 4; ++x) {
+        const float e0 = s[j >> 1][(j & 1) * 8 + 2 * x], e1 = s[j >> 1][(j & 1) * 8 + 2 * x + 1];
+        w[x] = pf_pack<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(e0, a.scale_log2, -ref)),
+                          __builtin_amdgcn_exp2f(__builtin_fmaf(e1, a.scale_log2, -ref)));
+        l = pf_add_pair<T>(w[x], l);
       }
       pb[j] = make_uint4(w[0], w[1], w[2], w[3]);
     }
-    psum += __shfl_xor(psum, 16);
-    psum += __shfl_xor(psum, 32);
-    l = l * alpha + psum;
-    // O^T += V^T P^T: dim block b, keys in the same order as pb
+    // O^T += V^T P^T: dim block b, 16-key step j
 #pragma unroll
-    for (int b = 0; b < DB; ++b) {
-      o[b] *= alpha;
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const char* vrow = vt_lds + (b * 16 + n) * VROW;
-        const uint2 lo = *reinterpret_cast<const uint2*>(vrow + ((2 * j) * 16 + g4 * 4) * 2);
-        const uint2 hi = *reinterpret_cast<const uint2*>(vrow + ((2 * j + 1) * 16 + g4 * 4) * 2);
-        o[b] = mfma16x16x32<T>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb[j], o[b]);
+      for (int b = 0; b < DB; ++b) {
+        const uint4 vf =
+            *reinterpret_cast<const uint4*>(vl + b * 32 * kVRow + pf_v_slot(b * 32 + n, 2 * j + half) * 16);
+        o[b] = mfma32x32x16<T>(vf, pb[j], o[b]);
       }
-    }
   }
-  if (!q_live) return;
+  l += __shfl_xor(l, 32);
+  if (query >= a.seq) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  char* op = a.out + ((int64_t)query * a.o_s + (int64_t)h * a.o_h) * T::bytes;
+  char* op = a.out + ((int64_t)query * a.o_s + (int64_t)h * a.o_h) * T::bytes + half * 8;
 #pragma unroll
-  for (int b = 0; b < DB; ++b) {  // this lane: dims b*16 + g4*4 .. +3 of its query
-    const uint32_t w0 = pf_pack<T>(o[b][0] * inv, o[b][1] * inv), w1 = pf_pack<T>(o[b][2] * inv, o[b][3] * inv);
-    *reinterpret_cast<uint2*>(op + (b * 16 + g4 * 4) * T::bytes) = make_uint2(w0, w1);
-  }
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {  // dims b*32 + x*8 + half*4 .. +3 of the lane's query
+      const uint32_t w0 = pf_pack<T>(o[b][4 * x] * inv, o[b][4 * x + 1] * inv);
+      const uint32_t w1 = pf_pack<T>(o[b][4 * x + 2] * inv, o[b][4 * x + 3] * inv);
+      *reinterpret_cast<uint2*>(op + b * 64 + x * 16) = make_uint2(w0, w1);
+    }
+}
+
+template <typename T, int D, int NW>
+static void launch_prefill(const PrefillArgs& a, const LaunchEvents& ev, hipStream_t s) {
+  const int64_t blocks = ((int64_t)a.seq + 32 * NW - 1) / (32 * NW) * a.q_heads;
+  launch(prefill_attention_kernel<T, D, NW>, dim3((unsigned)blocks), dim3(NW * kWave), 0, s, ev.start, ev.stop, a);
+}
+
+// Eight waves share each staged tile (one workgroup fills a CU) once there are
+// two such workgroups per CU to balance; below, four waves and up to two
+// workgroups per CU. us with eight / four waves, bf16, heads x head_dim:
+// 32768 tokens 32 x 128: 8597 / 9337; 4000 tokens 32 x 128: 159 / 169;
+// 4096 tokens 16 x 128 (256 eight-wave workgroups): 131 / 122; 1999 tokens
+// 28 x 128: 70 / 64; 1000 tokens 32 x 128: 37 / 32. Two waves lose
+// everywhere (1999 tokens: 93).
+template <typename T, int D>
+static void launch_prefill(const PrefillArgs& a, const LaunchEvents& ev, hipStream_t s) {
+  if (((int64_t)a.seq + 255) / 256 * a.q_heads >= 2 * kPfCUs)
+    launch_prefill<T, D, 8>(a, ev, s);
+  else
+    launch_prefill<T, D, 4>(a, ev, s);
 }
 
 }  // namespace nhs
@@ -290,18 +363,17 @@ extern "C" int nhs_prefill_attention(const void* q, int64_t q_seq_stride, int64_
   a.scale_log2 = (float)(1.4426950408889634 / sqrt((double)head_dim));
   a.out = static_cast<char*>(out);
   a.o_s = out_seq_stride, a.o_h = out_head_stride;
-  const dim3 grid((unsigned)((seq + kPfBM - 1) / kPfBM), (unsigned)q_heads), block(kPfThreads);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == NHS_BF16) {
     if (head_dim == 128)
-      launch(prefill_attention_kernel<BF16, 128>, grid, block, 0, s, ev.start, ev.stop, a);
+      launch_prefill<BF16, 128>(a, ev, s);
     else
-      launch(prefill_attention_kernel<BF16, 64>, grid, block, 0, s, ev.start, ev.stop, a);
+      launch_prefill<BF16, 64>(a, ev, s);
   } else {
     if (head_dim == 128)
-      launch(prefill_attention_kernel<F16, 128>, grid, block, 0, s, ev.start, ev.stop, a);
+      launch_prefill<F16, 128>(a, ev, s);
     else
-      launch(prefill_attention_kernel<F16, 64>, grid, block, 0, s, ev.start, ev.stop, a);
+      launch_prefill<F16, 64>(a, ev, s);
   }
   return launch_status(who);
 }
