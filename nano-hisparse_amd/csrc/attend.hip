@@ -36,7 +36,19 @@ namespace nhs {
 constexpr int kAttendThreads = 512;
 constexpr int kAttendWaves = kAttendThreads / kWave;
 constexpr int kMaxSplits = 32;
-constexpr int kMinRowsPerSplit = 32;
+constexpr int kMinRowsPerSplit = 32;  // the workspace holds partials for splits of this many rows
+// Fewest rows of a split, where fewer than one workgroup per CU leaves room
+// to split: a split costs the merge's store -> atomic -> load chain and every
+// further one lengthens the merge, while one workgroup reads several hundred
+// rows in a round trip or two. attend_kernel: four row groups of its eight
+// waves, at most kSplitRows. us at 32 rows per split / these, one request of
+// 4/2 heads of 64, fp32: 128 rows 8.8 / 5.2, 512 rows 16.2 / 7.0, 2048 rows
+// 25.6 / 10.6; 14/2 heads of 64, bf16, 2048 rows 35.1 / 15.2; 32/8 heads of
+// 128, fp32, 2048 rows 22.9 / 17.1 (half as many: 22.8; twice: 17.4).
+// attend_mfma_kernel (32/8 heads of 128, bf16, 128 rows per split / 256): 256
+// rows 9.4 / 7.3, 2048 rows 11.5 / 10.0 (512 rows per split: 12.0).
+constexpr int kSplitRows = 512;
+constexpr int kMSplitRows = 256;
 constexpr int kStage = 4096;  // row indices staged in LDS per pass (16 KiB)
 constexpr int kStagePerThread = kStage / kAttendThreads;
 constexpr int kIssueGroups = 2;  // row groups whose loads a wave issues together
@@ -1172,6 +1184,7 @@ extern "C" int nhs_attend_rows(const void* query, int32_t q_dtype, int64_t q_bat
     if (splits < 1) splits = 1;
     if (splits > max_splits_for(n_rows)) splits = max_splits_for(n_rows);
     if (splits > kMMaxSplits) splits = kMMaxSplits;
+    splits = std::min(splits, std::max(1, n_rows / kMSplitRows));
     const int block = kMTile * kMWaves;
     int per = (n_rows + splits - 1) / splits;
     per = (per + block - 1) / block * block;
@@ -1212,6 +1225,8 @@ extern "C" int nhs_attend_rows(const void* query, int32_t q_dtype, int64_t q_bat
   int splits = cus > 0 ? (cus + units / 2) / units : 1;
   if (splits < 1) splits = 1;
   if (splits > max_splits_for(n_rows)) splits = max_splits_for(n_rows);
+  const int group_rows = kAttendWaves * (kWave >> a.lpr_log2) * (C == 1 ? 4 : 2);  // U rows per lane slot
+  splits = std::min(splits, std::max(1, n_rows / std::min(4 * group_rows, kSplitRows)));
   if ((int64_t)units * splits > 0x7fffffff) return fail(NHS_ERR_UNSUPPORTED, "nhs_attend_rows: grid too large");
   a.kv_items = kv_items;
   a.n_splits = splits;
