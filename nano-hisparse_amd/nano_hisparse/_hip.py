@@ -131,6 +131,19 @@ def load(check_runtime: bool = True):
     return lib
 
 
+def load_launch():
+    """The native launchers (_launch.so), which call the loaded library."""
+    load()
+    try:
+        from . import _launch
+    except ImportError as exc:
+        raise RuntimeError(
+            f"the native launchers cannot be loaded ({exc}): build them with `make -C nano-hisparse_amd/csrc` "
+            "(or __graft_entry__.build())"
+        ) from exc
+    return _launch
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         message = _lib.nhs_last_error().decode(errors="replace") if _lib is not None else ""
