@@ -457,11 +457,37 @@ PyObject* select_resolve_batched(PyObject*, PyObject* const* a, Py_ssize_t nargs
   });
 }
 
+// ---- append ------------------------------------------------------------------------------------
+
+// nhs_append_page with the arguments row_kernels.PageAppender prepared (checked there), as whole numbers; returns the
+// status.
+PyObject* append_page(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 17) {
+    PyErr_SetString(PyExc_TypeError, "wrong number of arguments");
+    return nullptr;
+  }
+  int64_t v[17];
+  for (int i = 0; i < 17; ++i) {
+    v[i] = (int64_t)PyLong_AsUnsignedLongLong(a[i]);
+    if (PyErr_Occurred()) return nullptr;
+  }
+  const auto at = [&](int i) { return reinterpret_cast<void*>((uintptr_t)v[i]); };
+  int st;
+  {
+    NoGil free;
+    st = nhs_append_page(at(0), at(1), v[2], (int32_t)v[3], (int32_t)v[4], (int32_t)v[5], at(6), v[7], v[8],
+                         (int32_t)v[9], (int32_t)v[10], at(11), v[12], static_cast<float*>(at(13)), at(14), at(15),
+                         at(16));
+  }
+  return PyLong_FromLong(st);
+}
+
 #define NHS_METHOD(name) \
   { #name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr }
 PyMethodDef methods[] = {NHS_METHOD(linear_small_m), NHS_METHOD(linear_silu_mul),   NHS_METHOD(linear_rope),
                          NHS_METHOD(add_rmsnorm),    NHS_METHOD(attend_batched),    NHS_METHOD(prefill_attention),
-                         NHS_METHOD(quest_batched),  NHS_METHOD(select_resolve_batched), {nullptr, nullptr, 0, nullptr}};
+                         NHS_METHOD(quest_batched),  NHS_METHOD(select_resolve_batched),
+                         NHS_METHOD(append_page),    {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

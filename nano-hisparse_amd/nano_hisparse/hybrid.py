@@ -28,7 +28,7 @@ from __future__ import annotations
 import bisect
 import heapq
 from collections import Counter
-from contextlib import suppress
+from contextlib import contextmanager, nullcontext, suppress
 from dataclasses import dataclass, field
 from math import ceil
 
@@ -127,6 +127,24 @@ def store_entry(table, index, value):
     table[index : index + 1].fill_(value)
 
 
+def store_entries(table, entries):
+    """Write {index: value} into a device table on the current stream: one
+    upload per run of neighbouring indices, single fills for short runs."""
+    order = sorted(entries)
+    at = 0
+    while at < len(order):
+        end = at + 1
+        while end < len(order) and order[end] == order[end - 1] + 1:
+            end += 1
+        run = order[at:end]
+        if len(run) < 6:  # an upload costs the host about as much as six fills
+            for index in run:
+                store_entry(table, index, entries[index])
+        else:
+            table[run[0] : run[-1] + 1].copy_(upload([entries[i] for i in run], table.dtype, table.device))
+        at = end
+
+
 class HybridKVCache:
     def __init__(self, config, hot: HotConfig):
         if config.host_pages * config.page_size >= 2**31:
@@ -148,6 +166,7 @@ class HybridKVCache:
         self._awaiting_active: set = set()
         self._dormant: set = set()
         self._sweep = None  # (heap, rank cursor, group filter) while a tick runs
+        self._table_writes = None  # (layer tables, name) entries of a multi-page write or a release
         self._item_tables: dict = {}  # batch composition -> device nhs_layer_item table
         self.allocator = DeviceAllocator(config)
         self.storage = HostStore(config, self.allocator)
@@ -273,7 +292,7 @@ class HybridKVCache:
             self.storage.stats["append_resident_hits"] += 1
             return PageLease(self.storage, [page])
         slot = self._slot()
-        store_entry(self.tables[page.key[:2]].source, page.key[2], page.host_slot)
+        self._store_entry(page.key, "source", page.host_slot)
         self.storage.wait(self.storage.compute, self.allocator.slots[slot].fence)
         self._bind(page, slot, Location.RESIDENT)
         return None
@@ -281,16 +300,39 @@ class HybridKVCache:
     def _bind(self, page, slot, location):
         self.storage.bind(page, slot, location)
         group = page.key[:2]
-        store_entry(self.tables[group].resident, page.key[2], slot)
+        self._store_entry(page.key, "resident", slot)
         if group in self._awaiting:
             self._file(group)
 
-    def _detach(self, page):
-        self.storage.detach(page)
+    def _detach(self, page, fence=None):
+        self.storage.detach(page, fence)
         group = page.key[:2]
-        store_entry(self.tables[group].resident, page.key[2], -1)
+        self._store_entry(page.key, "resident", -1)
         if group in self._awaiting:
             self._file(group)
+
+    def _store_entry(self, key, name, value):
+        """One entry of a page's table, written now or, within
+        _collected_table_writes(), with the others at its end."""
+        if self._table_writes is None:
+            store_entry(getattr(self.tables[key[:2]], name), key[2], value)
+        else:
+            self._table_writes.setdefault((key[:2], name), {})[key[2]] = value
+
+    @contextmanager
+    def _collected_table_writes(self):
+        """Table entries written within are enqueued together at the end (the
+        last value of each): for operations over many pages during which
+        nothing enqueued reads the tables. Entries of layers released within
+        have no reader left and are dropped."""
+        self._table_writes = {}
+        try:
+            yield
+        finally:
+            writes, self._table_writes = self._table_writes, None
+            for (group, name), entries in writes.items():
+                if group in self.tables:
+                    store_entries(getattr(self.tables[group], name), entries)
 
     def _file(self, group):
         """Re-file an awaiting layer as active, dormant or neither (no
@@ -352,6 +394,8 @@ class HybridKVCache:
                 self.storage.stats["host_mirror_completions"] += 1
                 self._candidate(page)
             elif stream is not None:
+                if stream is self.storage.compute:  # a GPU cache's mirrors are all written on the compute stream
+                    break
                 blocked.add(stream)
 
     def _unpin_clean_pages(self, group):
@@ -546,7 +590,9 @@ class HybridKVCache:
         if self.tables[request_id, layer].busy:
             raise RuntimeError("cannot append during a row lease")
         try:
-            self.storage.append(request_id, layer, k, v, self._prepare_append, self._after_write)
+            # a prompt's pages: nothing between their placements reads the layer tables
+            with self._collected_table_writes() if len(k) > self.config.page_size else nullcontext():
+                self.storage.append(request_id, layer, k, v, self._prepare_append, self._after_write)
         finally:
             self._writing_key = None
 
@@ -653,26 +699,32 @@ class HybridKVCache:
         ):
             raise RuntimeError("cannot release a request with active row leases")
         store = self.storage
-        for tables in groups:
-            store.wait(store.transfer, tables.ready)
-            store.wait(store.transfer, tables.last_use)
+        # the transfer stream waits once for every user of the request's blocks; one fence behind them serves all
+        resident = [p for p in map(store.pages.__getitem__, store.requests[request_id].keys) if p.slot is not None]
+        waited = set()
+        fence = None
+        if store.cuda:
+            for tables in groups:
+                store.wait_each(store.transfer, (tables.ready, tables.last_use), waited)
+            for page in resident:
+                store.wait_each(store.transfer, store.users(page), waited)
             fence = store.event(store.transfer)
+        for tables in groups:
             for block in tables.blocks:
                 self.allocator.release(block, fence)
-        for key in store.requests[request_id].keys:
-            page = store.pages[key]
-            if page.slot is not None:
-                self._detach(page)
-        for key in [k for k in self._item_tables if request_id in k]:
-            del self._item_tables[key]  # its tensors go with the request
-        store.retire(request_id, keepalive=groups)
-        for key in [k for k in self.tables if k[0] == request_id]:
-            del self.tables[key]
-            del self._rank[key]
-            self._dirty.discard(key)
-            self._awaiting.discard(key)
-            self._awaiting_active.discard(key)
-            self._dormant.discard(key)
+        with self._collected_table_writes():  # the request's tables go with it: none is written
+            for page in resident:
+                self._detach(page, fence)
+            for key in [k for k in self._item_tables if request_id in k]:
+                del self._item_tables[key]  # its tensors go with the request
+            store.retire(request_id, keepalive=groups, waited=waited)
+            for key in [k for k in self.tables if k[0] == request_id]:
+                del self.tables[key]
+                del self._rank[key]
+                self._dirty.discard(key)
+                self._awaiting.discard(key)
+                self._awaiting_active.discard(key)
+                self._dormant.discard(key)
         self.collect(wait=wait)
 
     def collect(self, wait=False):

@@ -260,7 +260,7 @@ class PageAppender:
             raise ValueError("append_page: K/V rows must be contiguous with equal token strides")
         if host is not None and host.dtype != pool.dtype:
             raise ValueError("append_page: host and pool dtypes differ")
-        self.lib = _hip.load()
+        self.append_page = (_launch or _load_launch()).append_page
         self.k, self.v = k, v  # held for the write
         self.esize = k.element_size()
         self.k_ptr, self.v_ptr, self.token_stride = k.data_ptr(), v.data_ptr(), k.stride(0)
@@ -268,7 +268,7 @@ class PageAppender:
         self.pool_ptr, self.pool_stride = pool.data_ptr(), pool_block_stride(pool)
         self.host_ptr = host.data_ptr() if host is not None else 0
         self.sum_ptr, self.min_ptr, self.max_ptr = summaries.data_ptr(), minimum.data_ptr(), maximum.data_ptr()
-        self.stream = _stream(device)
+        self.stream = _raw_stream(_device_index(device))
 
     def __call__(self, first, count, block, within, host_page, bounds_index):
         """Rows first..first+count-1 of the write into rows within.. of pool
@@ -277,13 +277,11 @@ class PageAppender:
         if not (0 <= first and count >= 1 and first + count <= self.k.shape[0]):
             raise ValueError("append_page: rows outside the write")
         off = bounds_index * self.row_elems
-        status = self.lib.nhs_append_page(
-            ctypes.c_void_p(self.k_ptr + first * self.token_stride * self.esize),
-            ctypes.c_void_p(self.v_ptr + first * self.token_stride * self.esize), self.token_stride, self.dtype,
-            self.row_elems, self.page_size, ctypes.c_void_p(self.pool_ptr), self.pool_stride, int(block), int(within),
-            int(count), ctypes.c_void_p(self.host_ptr), int(host_page if self.host_ptr else 0),
-            ctypes.c_void_p(self.sum_ptr + off * 4), ctypes.c_void_p(self.min_ptr + off * self.esize),
-            ctypes.c_void_p(self.max_ptr + off * self.esize), self.stream,
+        row = first * self.token_stride * self.esize
+        status = self.append_page(
+            self.k_ptr + row, self.v_ptr + row, self.token_stride, self.dtype, self.row_elems, self.page_size,
+            self.pool_ptr, self.pool_stride, block, within, count, self.host_ptr, host_page if self.host_ptr else 0,
+            self.sum_ptr + off * 4, self.min_ptr + off * self.esize, self.max_ptr + off * self.esize, self.stream,
         )
         _hip.check(status, "nhs_append_page")
 

@@ -21,6 +21,7 @@ from enum import Enum
 from math import ceil
 
 import torch
+from torch._C import _cuda_getCurrentRawStream as _raw_stream
 
 from .allocator import DeviceAllocator
 from .config import CacheConfig, CapacityError
@@ -148,6 +149,7 @@ class HostStore:
 
             self.host_alias = MappedHost(self.host)
         self.compute = torch.cuda.current_stream(self.device) if self.cuda else None
+        self.page_bytes = self.pool[0].numel() * self.pool.element_size()
         self._capture_stream = None
         self.transfer = torch.cuda.Stream(device=self.device) if self.cuda else None
         self.pages: dict = {}
@@ -174,10 +176,6 @@ class HostStore:
     @property
     def owners(self):
         return [slot.owner for slot in self.allocator.slots]
-
-    @property
-    def page_bytes(self):
-        return self.pool[0].numel() * self.pool.element_size()
 
     @property
     def index_bytes(self):
@@ -225,7 +223,11 @@ class HostStore:
         return self._capture_stream if self._capture_stream is not None else self.compute
 
     def check_stream(self):
-        if self.cuda and torch.cuda.current_stream(self.device) not in (self.compute, self._capture_stream):
+        if not self.cuda:
+            return
+        current = _raw_stream(self.pool.get_device())  # a raw handle: this runs several times per page
+        if current != self.compute.cuda_stream and (
+                self._capture_stream is None or current != self._capture_stream.cuda_stream):
             raise RuntimeError("cache operations must use the construction compute stream")
 
     @contextlib.contextmanager
@@ -295,14 +297,30 @@ class HostStore:
         self.free_host.append(page.host_slot)
         self.stats["materialized_pages"] -= 1
 
-    def detach(self, page: Page):
-        """Drop a page's device block; reuse of the block waits on its events."""
+    def wait_each(self, stream, events, seen=None):
+        """Make `stream` wait for each distinct event (`seen`: the ids of
+        those it waits for already)."""
+        seen = set() if seen is None else seen
+        for ev in events:
+            if ev is not None and id(ev) not in seen:
+                seen.add(id(ev))
+                self.wait(stream, ev)
+
+    def users(self, page: Page):
+        """The events of a page's block and mirror: its write, its last
+        reader, its mirror and its layer's last batched read."""
+        return page.ready, page.last_use, page.host_ready, self.layer_reads.get(page.key[:2])
+
+    def detach(self, page: Page, fence=None):
+        """Drop a page's device block; reuse of the block waits on its
+        events, or on `fence`, an event recorded behind them."""
         assert self.pages.get(page.key) is page
         assert page.slot is not None and page.pins == 0
         assert page.host_enqueued_version == page.content_version
-        for ev in (page.ready, page.last_use, page.host_ready, self.layer_reads.get(page.key[:2])):
-            self.wait(self.transfer, ev)
-        self.allocator.release(page.slot, self.event(self.transfer))
+        if fence is None:
+            self.wait_each(self.transfer, self.users(page))
+            fence = self.event(self.transfer)
+        self.allocator.release(page.slot, fence)
         page.slot, page.location = None, Location.HOST
         self.resident_pages[page.key[:2]] -= 1
         self.stats["evictions"] += 1
@@ -348,10 +366,10 @@ class HostStore:
             # one kernel per page: pool rows, host mirror rows, bounds and summary
             appender = PageAppender(k.contiguous(), v.contiguous(), self.pool, self.host_alias, request.summaries,
                                     request.minimum, request.maximum)
-        done = 0
-        while done < len(k):
+        done, tokens = 0, len(k)
+        while done < tokens:
             index, within = divmod(start + done, P)
-            count = min(P - within, len(k) - done)
+            count = min(P - within, tokens - done)
             fresh = (request_id, layer, index) not in self.pages
             page = self.materialize(request_id, layer, index)
             try:
@@ -362,8 +380,7 @@ class HostStore:
                 raise
             if lease is not None:
                 lease.wait()
-            for ev in (page.ready, page.last_use, page.host_ready):
-                self.wait(self.compute, ev)  # earlier readers and mirrors of this page
+            self.wait_each(self.compute, (page.ready, page.last_use, page.host_ready))  # earlier readers and mirrors
             page.valid_tokens = within + count
             page.content_version += 1
             page.sealed = page.valid_tokens == P
@@ -415,19 +432,17 @@ class HostStore:
         if not self.cuda:
             page.host_committed_version = page.content_version
 
-    def retire(self, request_id, *, keepalive=()):
+    def retire(self, request_id, *, keepalive=(), waited=None):
+        """`waited`: ids of events the transfer stream waits for already."""
         self.check_stream()
         request = self.requests[request_id]
         if any(self.pages[key].pins for key in request.keys):
             raise RuntimeError("cannot free a request with active leases")
-        retired, waited = [], set()
+        retired, waited = [], set() if waited is None else waited
         for key in request.keys:
             page = self.pages[key]
             assert page.slot is None, "detach resident blocks before retiring host backing"
-            for ev in (page.ready, page.last_use, page.host_ready):
-                if ev is not None and id(ev) not in waited:  # pages of a batched step share events
-                    waited.add(id(ev))
-                    self.wait(self.transfer, ev)
+            self.wait_each(self.transfer, (page.ready, page.last_use, page.host_ready), waited)
             retired.append(self.pages.pop(key))
         del self.requests[request_id]
         for layer in range(request.layers):

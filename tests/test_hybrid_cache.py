@@ -320,3 +320,31 @@ def test_a_selection_of_8192_rows_resolves_and_attends(device):
     stats = cache.snapshot()["row_stats"]
     assert stats["resident_hits"] + stats["hot_hits"] + stats["misses"] == 2 * len(chosen)
     cache.assert_invariants()
+
+
+@pytest.mark.parametrize("tokens", [4, 5, 23, 24, 61])
+def test_tables_after_prompt_writes_hold_every_page(device, tokens):
+    """A prompt's table entries are written together at the end of its write
+    (one upload per run of pages, single entries for short runs): each
+    layer's tables then hold every page's host page and block, pages evicted
+    by later pages of the same or another layer included."""
+    hot = HotConfig(8, 8)
+    cfg = CacheConfig(gpu_pages=2 * hot.admission_blocks(4, 2) + 6, host_pages=96, page_size=4, kv_heads=1, head_dim=8,
+                      device=device)
+    cache = HybridKVCache(cfg, hot)
+    g = torch.Generator().manual_seed(tokens)
+    for rid in ("a", "b"):
+        cache.reserve(rid, tokens + 8, 2)
+    for part in (tokens, 3, 5):
+        for rid in ("a", "b"):
+            for layer in range(2):
+                kv = torch.randn(2, part, 1, 8, generator=g).to(device)
+                cache.write(rid, layer, kv[0], kv[1])
+                for (name, index), tables in cache.tables.items():
+                    pages = [cache.storage.pages.get((name, index, i)) for i in range(len(tables.source))]
+                    blocks = [-1 if p is None or p.slot is None else p.slot for p in pages]
+                    assert tables.source.tolist() == [-1 if p is None else p.host_slot for p in pages]
+                    assert tables.resident.tolist() == blocks
+        if part == 3:
+            cache.release_request("a")
+            cache.reserve("a", tokens + 8, 2)
