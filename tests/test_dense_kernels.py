@@ -118,3 +118,25 @@ def test_fused_batched_step_matches_per_request_decode(gpu, dtype, tol, micro_ba
         tokens = {n: int(batch[i].argmax()) for i, n in enumerate(prompts)}
     for c in caches:
         c.assert_invariants()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,heads,D,extra,offset", [
+    (3, 1, 16, 0, 0), (300, 32, 128, 0, 0), (2, 33, 128, 8, 0),  # one chunk; two and three workgroups per row
+    (3, 5, 24, 0, 0), (4, 3, 64, 4, 0), (4, 3, 64, 8, 2),  # halves, row strides and addresses off the 16-byte chunks
+])
+def test_rope_at_the_edges_of_its_chunks(gpu, dtype, rows, heads, D, extra, offset):
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    width = heads * D + extra
+    t = torch.randn(rows * width + offset, generator=g, device=gpu).to(dtype)[offset:].view(rows, width)
+    angle = torch.rand(rows, D // 2, generator=g, device=gpu) * 1000
+    cos, sin = angle.cos().to(dtype), angle.sin().to(dtype)
+    view = t[:, : heads * D].reshape(rows, heads, D)
+    c2, s2 = torch.cat((cos, cos), -1)[:, None, :], torch.cat((sin, sin), -1)[:, None, :]
+    lo, hi = view.chunk(2, -1)
+    want = view * c2 + torch.cat((-hi, lo), -1) * s2
+    tail = t[:, heads * D:].clone()
+    rk.rope_(t, heads, D, cos, sin)
+    assert torch.equal(t[:, : heads * D].reshape(rows, heads, D), want)
+    assert torch.equal(t[:, heads * D:], tail)
