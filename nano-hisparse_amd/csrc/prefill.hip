@@ -2,8 +2,10 @@
 //
 // out[s, h] = softmax_{t <= s}(q[s, h] . k[t, h/g] * D^-1/2) . v[t, h/g] for
 // one prompt of `seq` tokens, bf16 or fp16 in, fp32 accumulation. A
-// workgroup of NW waves owns 32 * NW queries of one query head (32 per wave)
-// and walks the key tiles of 64 up to the diagonal with an online softmax.
+// workgroup of 8 waves takes 256 queries of one query head (32 per wave) and
+// walks the key tiles of 64 up to the diagonal with an online softmax; or
+// (KSPLIT 2, where that leaves the chip idle) 128 queries, the two halves of
+// the workgroup taking the even and the odd tiles, whose sums meet in LDS.
 //
 // MFMA v_mfma_f32_32x32x16 (bf16 / f16): lane l supplies row l%32 of A and
 // column l%32 of B at k = (l/32)*8 .. +7, and receives D rows
@@ -14,18 +16,20 @@
 // statistics live in the lane pair l, l ^ 32. The output is accumulated
 // transposed too, O^T = V^T P^T: registers 8s .. 8s+7 of a score block are
 // the B operand of k step s as they stand once the step's 16 keys are taken
-// in the order (l/32)*4 + 0..3, 8 + (l/32)*4 + 0..3, and the LDS V^T tile
-// stores each 16 keys in that order, so its A operand is one 16-byte read.
-// The rescaling by a query's max stays in its lane.
+// in the order (l/32)*4 + 0..3, 8 + (l/32)*4 + 0..3, and the transposing LDS
+// read (ds_read_b64_tr_b16: four keys of one dim per lane from row-major V)
+// fetches the A operand in that order. The rescaling by a query's max stays
+// in its lane.
 //
 // Why 32 queries per wave and 32x32 tiles: a wave reads every K and V byte
 // of the tile from LDS once per MFMA operand, so the LDS bytes per flop fall
 // with the queries a wave holds. At 16 per wave (16x16 tiles) the LDS reads
 // took twice the matrix cores' time; at 32 they take as long as it does, and
 // the wave still fits 256 registers, so two waves share a SIMD and one's
-// softmax runs beside the other's MFMAs. K and V^T rows are stored with their
-// 16-byte chunks permuted by an XOR of the row, so that reads of 16 rows at
-// one chunk meet all 64 banks.
+// softmax runs beside the other's MFMAs. Tiles go from global memory straight
+// to LDS; the 16-byte chunks of their rows are permuted by an XOR of the row
+// (the lanes of a load fetch the chunks in that order), so that the rows of a
+// read meet distinct banks.
 //
 // The weights are rounded to the input dtype for the P.V product and the
 // denominator sums the same rounded weights, so each output is an exact
@@ -34,11 +38,11 @@
 // more, 3% of the time at 32K tokens, but the largest weight would no longer
 // be exactly 1: the error against float64 grew by 3%.)
 //
-// Measured (MI355X, bf16, 32/8 heads of 128): 32768 tokens 8.86 ms, 993
-// TFLOP/s causal (22.37 ms with 16 queries per wave and 16x16 tiles; a large
-// hipBLASLt product reaches 1342); 4000 tokens 157 us (605); 1999 tokens of
-// 28/4 heads 63 us (159), where the longest workgroup's 32 tiles of ~2 us
-// are the bound and the chip is half idle.
+// Measured (MI355X, bf16, 32/8 heads of 128): 32768 tokens 7.8-8.3 ms, 1060
+// to 1130 TFLOP/s causal (22.37 ms with 16 queries per wave and 16x16 tiles, 8.86 with
+// tiles staged through registers and V transposed by the stores; a large
+// hipBLASLt product reaches 1342); 4000 tokens 146 us (605, 157); 1999 tokens
+// of 28/4 heads 46 us (159, 63); 333 tokens 11.7 us (19.7, 14.9).
 #include <math.h>
 
 #include "nhs_common.h"
@@ -46,7 +50,12 @@
 namespace nhs {
 
 constexpr int kPfBN = 64;            // keys per tile
-constexpr int kPfCUs = 256;
+constexpr int kPfWaves = 8, kPfThreads = kPfWaves * kWave;
+// Workgroups of 256 queries from which each takes every tile. us with one /
+// two shares (bf16, heads x head_dim): 4096 tokens 16 x 128 (256 of them) 116
+// / 88, 6000 tokens (384) 181 / 186, 8192 tokens (512) 285 / 312; 4096 tokens
+// 32 x 64 (512) 102 / 90, 16384 tokens 16 x 64 (1024) 584 / 606.
+constexpr int pf_whole(int head_dim) { return head_dim == 128 ? 384 : 768; }
 
 typedef __bf16 pf_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_f16x8 __attribute__((ext_vector_type(8)));
@@ -86,10 +95,6 @@ __device__ __forceinline__ float pf_add_pair(uint32_t pair, float acc) {
                                   false);
 }
 
-__device__ __forceinline__ uint32_t pf_word(const uint4& v, int w) {
-  return w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w;
-}
-
 struct PrefillArgs {
   const char* q;
   const char* k;
@@ -101,30 +106,53 @@ struct PrefillArgs {
   int64_t o_s, o_h;
 };
 
-// LDS slot of 16-byte chunk c of K row r (D * 2 bytes) and of V^T row r (128 bytes): any 16 consecutive rows at one
-// chunk fall on distinct banks.
+// LDS slot of 16-byte chunk c of K row r: any 16 consecutive rows at one chunk fall on distinct banks
 template <int D>
 __device__ __forceinline__ int pf_k_slot(int r, int c) {
   return D == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7);
 }
-__device__ __forceinline__ int pf_v_slot(int r, int c) { return c ^ (((r >> 1) ^ (r >> 4)) & 7); }
+// and of V row (key) r: the 4 rows of a transposing read fall on distinct banks
+template <int D>
+__device__ __forceinline__ int pf_v_slot(int r, int c) {
+  return D == 128 ? c ^ (4 * (r & 3)) : c ^ (4 * ((r >> 1) & 1));
+}
 
-template <typename T, int D, int NW>
-__global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(PrefillArgs a) {
-  constexpr int kThreads = NW * kWave;
-  constexpr int BM = 32 * NW;          // queries per workgroup
+constexpr int kPfVmcnt0 = 0x0f70;  // s_waitcnt vmcnt(0), the other counters left alone
+
+// 16 bytes per lane from global memory to LDS at `dst` (uniform over the wave) + 16 * lane
+__device__ __forceinline__ void pf_load_lds(const char* src, char* dst) {
+  __builtin_amdgcn_global_load_lds((const NHS_GLOBAL void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+typedef short pf_i16x4 __attribute__((ext_vector_type(4)));
+
+// Transposing read: of each 16 lanes, lanes 4r .. 4r+3 name 16 elements of row r; lane i receives column i of the four
+// rows.
+__device__ __forceinline__ uint2 pf_read_tr(const char* p) {
+  return __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_i16x4*)const_cast<char*>(p)));
+}
+
+template <typename T, int D, int KSPLIT>
+__global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillArgs a) {
+  constexpr int kThreads = kPfThreads;
+  constexpr int QW = kPfWaves / KSPLIT;  // waves of different queries
+  constexpr int BM = 32 * QW;            // queries per workgroup
   constexpr int KS = D / 16;           // 16-wide k steps of Q.K
   constexpr int DB = D / 32;           // 32-wide dim blocks of the output
   constexpr int C = D / 8;             // 16-byte chunks of a K or V row
-  constexpr int kVRow = kPfBN * 2;     // bytes per V^T row
-  // a staging unit is four 16-byte loads: 4 keys x 8 dims of V (a 4-key piece of 8 V^T rows), or one chunk of 4 K rows
-  constexpr int kUnits = kPfBN * D / 32;  // units per tile of each
-  constexpr int kMine = (2 * kUnits + kThreads - 1) / kThreads;
-  // two buffers per tile: tile t+1 is stored while tile t is read, one barrier per tile
-  __shared__ __attribute__((aligned(16))) char k_buf[2][kPfBN * D * 2];
-  __shared__ __attribute__((aligned(16))) char v_buf[2][D * kVRow];
+  // Tiles go straight to LDS (global_load_lds, 1 KB per wave and instruction: kRows rows). Two buffers of their own
+  // names, used by alternate rounds: the compiler then knows that reads of one need not wait for loads into the other.
+  constexpr int kRows = 1024 / (D * 2);
+  constexpr int kInstr = kPfBN / kRows;             // instructions per tile
+  constexpr int kMine = kInstr * KSPLIT / kPfWaves;  // of a wave, per round, for K and for V each
+  constexpr int kTile = kPfBN * D * 2;              // bytes
+  __shared__ __attribute__((aligned(16))) char k0[KSPLIT * kTile], k1[KSPLIT * kTile];
+  __shared__ __attribute__((aligned(16))) char v0[KSPLIT * kTile], v1[KSPLIT * kTile];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_id % QW, share = wave_id / QW;  // the wave's queries, its tile of each round
   const int half = lane >> 5, n = lane & 31;
   // The longest rows first; with a multiple of 8 heads each XCD (workgroup id mod 8) keeps neighbouring heads, so that
   // the heads of one KV head read its tiles from one L2.
@@ -153,79 +181,59 @@ __global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(Prefill
     for (int i = 0; i < 16; ++i) o[b][i] = 0.f;
 
   const int last_key = min(a.seq, q0 + BM) - 1;
-  const int n_tiles = last_key / kPfBN + 1;
+  const int n_rounds = last_key / (kPfBN * KSPLIT) + 1;
   const char* kbase = a.k + (int64_t)kvh * a.k_h * T::bytes;
   const char* vbase = a.v + (int64_t)kvh * a.v_h * T::bytes;
-  uint4 reg[kMine][4];
-  auto load_tile = [&](int t0) {
+  // this lane's part of load i: row `row` of its tile (below), chunk of the row, permuted so that the LDS slots come
+  // out in lane order
+  const int lrow = lane / C;
+  const int k_chunk = pf_k_slot<D>(wave_id * kRows + lrow, lane % C), v_chunk = pf_v_slot<D>(lrow, lane % C);
+  constexpr int kRound = kPfBN * KSPLIT;
+  const int64_t k_stride = a.k_s * T::bytes, v_stride = a.v_s * T::bytes;
+  const char* kp[kMine];
+  const char* vp[kMine];
 #pragma unroll
-    for (int u = 0; u < kMine; ++u) {
-      const int unit = tid + u * kThreads;
-      const bool is_v = unit < kUnits;
-      if (unit >= 2 * kUnits) break;
-      const int x = is_v ? unit : unit - kUnits;
-      const int row = is_v ? (x / C) * 4 : x / C, step = is_v ? 1 : kPfBN / 4;
-      const char* base = (is_v ? vbase : kbase) + (x % C) * 16;
-      const int64_t stride = (is_v ? a.v_s : a.k_s) * T::bytes;
-      if (t0 + kPfBN <= a.seq) {
-        const char* p = base + (int64_t)(t0 + row) * stride;
+  for (int i = 0; i < kMine; ++i) {
+    const int row = (i * kPfWaves + wave_id) * kRows + lrow;  // of the round (its tiles one after another)
+    kp[i] = kbase + k_chunk * 16 + row * k_stride;
+    vp[i] = vbase + v_chunk * 16 + row * v_stride;
+  }
+  auto load_round = [&](int t, char* kb, char* vb) {
+    const bool whole = (t + 1) * kRound <= a.seq;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) reg[u][i] = *reinterpret_cast<const uint4*>(p + i * step * stride);
-      } else {  // rows past the end re-read the last key (masked below)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          reg[u][i] = *reinterpret_cast<const uint4*>(base + (int64_t)min(t0 + row + i * step, a.seq - 1) * stride);
+    for (int i = 0; i < kMine; ++i) {
+      const int dst = (i * kPfWaves + wave_id) * 1024;
+      const char* ks = kp[i];
+      const char* vs = vp[i];
+      if (!whole) {  // rows past the end re-read the last key (masked below)
+        const int row = min(t * kRound + (i * kPfWaves + wave_id) * kRows + lrow, a.seq - 1);
+        ks = kbase + k_chunk * 16 + row * k_stride;
+        vs = vbase + v_chunk * 16 + row * v_stride;
       }
+      pf_load_lds(ks, kb + dst);
+      pf_load_lds(vs, vb + dst);
+      kp[i] += kRound * k_stride;
+      vp[i] += kRound * v_stride;
     }
   };
-  auto store_tile = [&](int buf) {
+  // addresses within a tile: K row n at k step st, V^T's two 4-key pieces of dim block b
+  const int k_row = n * (D * 2);
+  const int j = (lane & 15) >> 2;
+  int v_at[DB];
 #pragma unroll
-    for (int u = 0; u < kMine; ++u) {
-      const int unit = tid + u * kThreads;
-      if (unit >= 2 * kUnits) break;
-      if (unit < kUnits) {
-        const int kg = unit / C, r0 = (unit % C) * 8;  // keys 4 kg .. +3, dims r0 .. +7
-        const int c = 2 * (kg >> 2) + (kg & 1), piece = (kg >> 1) & 1;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-          const uint32_t lo = __builtin_amdgcn_perm(pf_word(reg[u][1], j >> 1), pf_word(reg[u][0], j >> 1), sel);
-          const uint32_t hi = __builtin_amdgcn_perm(pf_word(reg[u][3], j >> 1), pf_word(reg[u][2], j >> 1), sel);
-          *reinterpret_cast<uint2*>(v_buf[buf] + (r0 + j) * kVRow + pf_v_slot(r0 + j, c) * 16 + piece * 8) =
-              make_uint2(lo, hi);
-        }
-      } else {
-        const int x = unit - kUnits, c = x % C;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = x / C + i * (kPfBN / 4);
-          *reinterpret_cast<uint4*>(k_buf[buf] + r * (D * 2) + pf_k_slot<D>(r, c) * 16) = reg[u][i];
-        }
-      }
-    }
-  };
+  for (int b = 0; b < DB; ++b)
+    v_at[b] = (4 * half + j) * (D * 2) + pf_v_slot<D>(j, b * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) * 16 + (lane & 1) * 8;
 
-  auto stage = [&](int t) {
-    store_tile((t + 1) & 1);
-    if (t + 2 < n_tiles) load_tile((t + 2) * kPfBN);  // in flight during the rest of tile t's math and tile t+1's QK
-  };
-
-  load_tile(0);
-  store_tile(0);
-  if (n_tiles > 1) load_tile(kPfBN);
-  for (int t = 0; t < n_tiles; ++t) {
-    const int t0 = t * kPfBN;
-    // tile t's buffer is complete and every wave is done with tile t-1's
-    // buffer, which takes tile t+1 (loaded during tile t-1's math)
+  auto round = [&](int t, char* kb, char* vb, char* kb_next, char* vb_next) {
+    const int t0 = t * kRound + share * kPfBN;
+    // this wave's loads of round t are in; after the barrier every wave's are, and every wave is done with the other
+    // buffers, which take round t+1
+    __builtin_amdgcn_s_waitcnt(kPfVmcnt0);
     __syncthreads();
-    // the next tile is stored under the first MFMAs (waves without queries in this tile store it alone)
-    const bool stages = t + 1 < n_tiles;
-    if (t0 > wq0 + 31) {  // wholly above the wave's diagonal
-      if (stages) stage(t);
-      continue;
-    }
-    const char* kl = k_buf[t & 1] + n * (D * 2);
-    const char* vl = v_buf[t & 1] + n * kVRow;
+    if (t + 1 < n_rounds) load_round(t + 1, kb_next, vb_next);
+    if (t0 > min(wq0 + 31, last_key)) return;  // wholly above the wave's diagonal or past the last key
+    const char* kl = kb + share * kTile + k_row;
+    const char* vl = vb + share * kTile;
 
     // S^T for 2 key blocks of 32: s[kb][i] holds key t0 + kb*32 + (i/4)*8 + half*4 + i%4
     pf_f32x16 s[2];
@@ -241,7 +249,15 @@ __global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(Prefill
             *reinterpret_cast<const uint4*>(kl + kb * 32 * D * 2 + pf_k_slot<D>(n, 2 * st + half) * 16);
         s[kb] = mfma32x32x16<T>(kf, qf[st], s[kb]);
       }
-    if (stages) stage(t);
+    if constexpr (D == 128) {  // keep eight K reads ahead of the MFMAs (two by default: 3% slower)
+      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
+    }
     // causal and past-the-end mask (a tile wholly below the wave's diagonal
     // and inside the prompt needs none)
     if (t0 + kPfBN - 1 > wq0 || t0 + kPfBN > a.seq) {  // uniform over the wave
@@ -289,12 +305,44 @@ __global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(Prefill
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int b = 0; b < DB; ++b) {
-        const uint4 vf =
-            *reinterpret_cast<const uint4*>(vl + b * 32 * kVRow + pf_v_slot(b * 32 + n, 2 * j + half) * 16);
+        const uint2 lo = pf_read_tr(vl + v_at[b] + (16 * j) * (D * 2));
+        const uint2 hi = pf_read_tr(vl + v_at[b] + (16 * j + 8) * (D * 2));
+        const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
         o[b] = mfma32x32x16<T>(vf, pb[j], o[b]);
       }
+  };
+  load_round(0, k0, v0);
+  for (int t = 0; t < n_rounds; t += 2) {
+    round(t, k0, v0, k1, v1);
+    if (t + 1 < n_rounds) round(t + 1, k1, v1, k0, v0);
   }
   l += __shfl_xor(l, 32);
+  if constexpr (KSPLIT == 2) {
+    // the waves of the second share hand their sums over through the tile buffers (registers by lane: each lane's
+    // partner holds the same query and dims)
+    float* part = reinterpret_cast<float*>(wave < QW / 2 ? k0 : k1) + wave % (QW / 2) * (DB * 16 * kWave) + lane;
+    float* stat = reinterpret_cast<float*>(v0) + wave * 2 * kWave + lane;
+    __syncthreads();
+    if (share) {
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(b * 16 + i) * kWave] = o[b][i];
+      stat[0] = m;
+      stat[kWave] = l;
+    }
+    __syncthreads();
+    if (share) return;
+    const float m2 = stat[0], l2 = stat[kWave];
+    const float both = fmaxf(m, m2), ref = both == -INFINITY ? 0.f : both;
+    const float f1 = __builtin_amdgcn_exp2f((m - ref) * a.scale_log2);
+    const float f2 = __builtin_amdgcn_exp2f((m2 - ref) * a.scale_log2);
+    l = l * f1 + l2 * f2;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[b][i] = o[b][i] * f1 + part[(b * 16 + i) * kWave] * f2;
+  }
   if (query >= a.seq) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
   char* op = a.out + ((int64_t)query * a.o_s + (int64_t)h * a.o_h) * T::bytes + half * 8;
@@ -308,25 +356,19 @@ __global__ __launch_bounds__(NW* kWave, 2) void prefill_attention_kernel(Prefill
     }
 }
 
-template <typename T, int D, int NW>
+template <typename T, int D, int KSPLIT>
 static void launch_prefill(const PrefillArgs& a, const LaunchEvents& ev, hipStream_t s) {
-  const int64_t blocks = ((int64_t)a.seq + 32 * NW - 1) / (32 * NW) * a.q_heads;
-  launch(prefill_attention_kernel<T, D, NW>, dim3((unsigned)blocks), dim3(NW * kWave), 0, s, ev.start, ev.stop, a);
+  constexpr int BM = 32 * kPfWaves / KSPLIT;
+  const int64_t blocks = ((int64_t)a.seq + BM - 1) / BM * a.q_heads;
+  launch(prefill_attention_kernel<T, D, KSPLIT>, dim3((unsigned)blocks), dim3(kPfThreads), 0, s, ev.start, ev.stop, a);
 }
 
-// Eight waves share each staged tile (one workgroup fills a CU) once there are
-// two such workgroups per CU to balance; below, four waves and up to two
-// workgroups per CU. us with eight / four waves, bf16, heads x head_dim:
-// 32768 tokens 32 x 128: 8597 / 9337; 4000 tokens 32 x 128: 159 / 169;
-// 4096 tokens 16 x 128 (256 eight-wave workgroups): 131 / 122; 1999 tokens
-// 28 x 128: 70 / 64; 1000 tokens 32 x 128: 37 / 32. Two waves lose
-// everywhere (1999 tokens: 93).
 template <typename T, int D>
 static void launch_prefill(const PrefillArgs& a, const LaunchEvents& ev, hipStream_t s) {
-  if (((int64_t)a.seq + 255) / 256 * a.q_heads >= 2 * kPfCUs)
-    launch_prefill<T, D, 8>(a, ev, s);
+  if (((int64_t)a.seq + 255) / 256 * a.q_heads >= pf_whole(D))
+    launch_prefill<T, D, 1>(a, ev, s);
   else
-    launch_prefill<T, D, 4>(a, ev, s);
+    launch_prefill<T, D, 2>(a, ev, s);
 }
 
 }  // namespace nhs

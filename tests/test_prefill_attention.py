@@ -77,3 +77,38 @@ def test_model_prefill_runs_the_flash_kernel(gpu, dtype, monkeypatch):
     want = model.prefill(tokens)
     err = (got - want).abs().max().item()
     assert err <= 5e-2 * max(1.0, want.abs().max().item()), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,Hq,Hkv,D", [
+    # rounds of two 64-key tiles, workgroups of 128 queries: one tile short of, at and past their edges
+    (63, 8, 2, 128), (127, 3, 1, 64), (128, 3, 1, 128), (129, 8, 2, 64), (191, 5, 5, 128), (193, 2, 2, 64),
+    (255, 1, 1, 128), (257, 28, 4, 128), (384, 14, 2, 64), (641, 4, 2, 64),
+    # enough workgroups of 256 queries that each takes every tile
+    (769, 128, 4, 128), (1025, 96, 8, 64), (3073, 32, 8, 128),
+])
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2e-2), (torch.float16, 1e-2)])
+def test_prefill_attention_at_the_edges_of_tiles_and_rounds(gpu, dtype, tol, S, Hq, Hkv, D):
+    test_prefill_attention_matches_fp32_reference(gpu, dtype, tol, S, Hq, Hkv, D)
+
+
+@pytest.mark.gpu
+def test_prefill_attention_of_infinite_and_nan_scores(gpu):
+    """A query that is NaN or meets an infinite score is NaN as in the dense
+    softmax, and the queries before the key that is infinite are untouched;
+    keys whose scores are -inf carry no weight."""
+    g = torch.Generator(device=gpu).manual_seed(9)
+    S, Hq, Hkv, D = 300, 2, 1, 64
+    q, k, v = (torch.randn(S, h, D, generator=g, device=gpu).half() for h in (Hq, Hkv, Hkv))
+    q[10, 0, 0] = float("nan")
+    q[:, 1, 3] = q[:, 1, 3].abs() + 0.5
+    k[200, 0] = 0
+    k[200, 0, 3] = float("-inf")  # -inf for head 1's queries (0 * inf is not met: the rest of the key is finite)
+    q[:, 0, 3] = -q[:, 0, 3].abs() - 0.5  # +inf for head 0's
+    out = rk.prefill_attention(q, k, v)
+    want = reference(q, k, v)
+    for h in (0, 1):
+        a, b = out[:, h].float(), want[:, h]
+        assert torch.equal(a.isnan(), b.isnan())
+        assert (a - b)[~b.isnan()].abs().max().item() <= 1e-2
+    assert out[10, 0].isnan().all() and out[200:, 0].isnan().all() and not out[:, 1].isnan().any()
