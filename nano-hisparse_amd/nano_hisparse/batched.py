@@ -76,6 +76,8 @@ class BatchDecode:
         self.layers = store.requests[ids[0]].layers
         self.items = cache._layer_items(ids)
         self.max_pages = max(store.requests[r].page_count for r in ids)
+        self.max_tokens = max(store.requests[r].max_tokens for r in ids)  # the step's positions are below
+        self.workspace = None  # the attention's, where the stream's own does not serve (make_workspace)
         both = torch.tensor([lengths, [n + 1 for n in lengths]], dtype=torch.int64).pin_memory()
         if lengths_buffer is None:
             self.dev_lengths = both.to(cache.device, non_blocking=True)
@@ -162,6 +164,15 @@ class BatchDecode:
         self._written.extend(pages)
         store.stats["d2h_bytes"] += row_bytes * len(self.ids)
         self._appended.add(layer)
+
+    def make_workspace(self, q_heads, top_pages):
+        """Give the step an attention workspace of its own, cleared now: a
+        captured step's workspace is read by every replay, beside whatever
+        else runs with the capture stream's."""
+        cfg = self.cache.config
+        need = rk._hip.load().nhs_attend_workspace_bytes(len(self.ids), q_heads, cfg.head_dim,
+                                                         top_pages * cfg.page_size)
+        self.workspace = torch.zeros(need, dtype=torch.uint8, device=self.cache.device)
 
     def sync_tables(self):
         """Make the compute stream wait for every pending event of the batch's
@@ -292,7 +303,7 @@ class BatchDecode:
         layer, query, physical, gathered = handle
         cache, store = self.cache, self.cache.storage
         store.wait(store.active_compute(), gathered)
-        out = rk.attend_batched(query, cache.pool, physical, cache.config.page_size)
+        out = rk.attend_batched(query, cache.pool, physical, cache.config.page_size, workspace=self.workspace)
         self._attended.add(layer)
         return out
 

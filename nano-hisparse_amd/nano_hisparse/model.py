@@ -12,6 +12,7 @@ state dicts load either way and a seeded random init draws the same weights.
 from __future__ import annotations
 
 from dataclasses import dataclass
+from typing import NamedTuple
 
 import torch
 from torch import nn
@@ -19,6 +20,9 @@ from torch.nn import functional as F
 
 from .selection import Selection, quest_selection, select_pages
 from .storage import upload
+
+
+ROPE_TABLE_ROWS = 1 << 17  # longest cos/sin tables a model keeps (32 MB at head_dim 128 in 16 bits)
 
 
 @dataclass
@@ -206,9 +210,7 @@ class Model(nn.Module):
 
         cfg, n = self.config, len(x)
         D, Hq, Hkv = cfg.head_dim, cfg.num_attention_heads, cfg.num_key_value_heads
-        inv_freq = cfg.rope_theta ** (-torch.arange(0, D, 2, device=x.device).float() / D)
-        angle = torch.arange(n, device=x.device).float()[:, None] * inv_freq[None, :]
-        cos, sin = angle.cos().to(x.dtype), angle.sin().to(x.dtype)
+        cos, sin = _rope_rows(cfg, torch.arange(n, device=x.device), x.dtype)
         x, delta = x.contiguous(), None
         for index, layer in enumerate(self.model.layers):
             attn, norm1, norm2 = layer.self_attn, layer.input_layernorm, layer.post_attention_layernorm
@@ -221,7 +223,8 @@ class Model(nn.Module):
                 cache.write(request_id, index, k, v)
             o = attn.o_proj(rk.prefill_attention(q, k, v).reshape(n, -1)).contiguous()
             delta = layer.mlp(rk.add_rmsnorm(x, o, norm2.weight, _eps(norm2, cfg))).contiguous()
-        return self.lm_head(self.model.norm(x[-1] + delta[-1])).float()
+        last = _Last(x[-1:], delta[-1:])
+        return _linear(self._final_norm([last]), self.lm_head.weight, self.lm_head.bias)[0].float()
 
     @torch.inference_mode()
     def decode(self, token: int, request_id, cache, top_k=None, backend="auto", selector="quest"):
@@ -347,9 +350,39 @@ class Model(nn.Module):
                         b.pre(index + 1, layers[index + 1], fused[index + 1], top_k)
             finally:
                 rk.set_gather_workgroups(0)
-        x = groups[0].x + groups[0].delta if len(groups) == 1 else torch.cat([g.x + g.delta for g in groups])
-        return _linear(self.model.norm(x), self.lm_head.weight, self.lm_head.bias).float()
+        return _linear(self._final_norm(groups), self.lm_head.weight, self.lm_head.bias).float()
 
+    def _final_norm(self, groups):
+        """The last residual add and norm of every group's rows."""
+        from . import row_kernels as rk
+
+        norm = self.model.norm
+        if norm.weight.dtype == self.dtype and norm.weight.is_contiguous():
+            rows = [rk.add_rmsnorm(g.x, g.delta, norm.weight, _eps(norm, self.config), write_back=False)
+                    for g in groups]
+        else:
+            rows = [norm(g.x + g.delta) for g in groups]
+        return rows[0] if len(rows) == 1 else torch.cat(rows)
+
+    def _rope_tables(self, limit):
+        """cos and sin [rows, head_dim / 2] in the model dtype of every
+        position below `limit` (None beyond ROPE_TABLE_ROWS positions): kept
+        with the model, longer ones (twice as long each) made on demand. A decode step
+        then reads its rows instead of computing them in eleven launches."""
+        if limit > ROPE_TABLE_ROWS:
+            return None
+        cfg = self.config
+        key = (self.device, self.dtype, cfg.rope_theta, cfg.head_dim)
+        made = self.__dict__.setdefault("_rope", [])  # every table made: other streams may still read the shorter ones
+        for kept, tables in reversed(made):
+            if kept == key and len(tables[0]) >= limit:
+                return tables
+        rows = min(ROPE_TABLE_ROWS, max(4096, 1 << (limit - 1).bit_length()))
+        tables = _rope_rows(cfg, torch.arange(rows, device=self.device), self.dtype)
+        if self.device.type == "cuda":
+            torch.cuda.current_stream(self.device).synchronize()  # complete for every stream from here on
+        made.append((key, tables))
+        return tables
 
     def clear_decode_graphs(self):
         """Drops every captured decode-step graph, with the cache, buffers and
@@ -407,9 +440,15 @@ class Model(nn.Module):
             # Fuse before the capture: a fusion inside it would be recorded and not run, and every replay would
             # read the separate weights, which fusing frees.
             self._fused_projections()
+            # The same holds for cos/sin tables made inside it, and a workspace made inside it would be cleared by
+            # every replay.
+            limit = max(cache.storage.requests[r].max_tokens for r in request_ids)
+            tables = self._rope_tables(limit)
             buffers = [(torch.empty(2, b - a, dtype=torch.int64, device=cache.device),
                         torch.empty(b - a, dtype=torch.int64, device=cache.device)) for a, b in spans]
             steps = open_steps(buffers)
+            for step in steps:
+                step.make_workspace(self.config.num_attention_heads, top_k)
             graph = torch.cuda.CUDAGraph()
             side = torch.cuda.Stream(device=cache.device)
             side.wait_stream(store.compute)
@@ -421,10 +460,9 @@ class Model(nn.Module):
                 logits = self._run_groups(groups, top_k)
             for step in steps:
                 step.forget_capture_events()
-            # the capture stream lives as long as the graph: buffers cached per stream during the capture
-            # (the attention workspace) belong to the graph's memory
+            # what the graph reads outside its own memory lives as long as it does
             entry = {"cache": cache, "items": items, "buffers": buffers, "graph": graph, "logits": logits,
-                     "stream": side}
+                     "stream": side, "tables": tables, "workspaces": [step.workspace for step in steps]}
             graphs[key] = entry
             while len(graphs) > 8:  # the most recent compositions keep their graphs
                 del graphs[next(iter(graphs))]
@@ -438,6 +476,13 @@ class Model(nn.Module):
         return entry["logits"].clone()
 
 
+class _Last(NamedTuple):
+    """A prompt's last row, as _final_norm takes a group."""
+
+    x: torch.Tensor
+    delta: torch.Tensor
+
+
 class _Group:
     """One batch group of decode_batch: its residual stream, RoPE tables,
     cache step and the gather handle in flight."""
@@ -446,12 +491,12 @@ class _Group:
         cfg = model.config
         self.model, self.cfg = model, cfg
         self.step = cache.decode_batch(request_ids, overlap) if step is None else step
-        D = cfg.head_dim
         positions = self.step.dev_lengths[0]  # already on the device
-        inv_freq = cfg.rope_theta ** (-torch.arange(0, D, 2, device=model.device).float() / D)
-        angle = positions.float()[:, None] * inv_freq[None, :]
-        self.cos = angle.cos().to(model.dtype).contiguous()
-        self.sin = angle.sin().to(model.dtype).contiguous()
+        tables = model._rope_tables(self.step.max_tokens)
+        if tables is None:
+            self.cos, self.sin = _rope_rows(cfg, positions, model.dtype)
+        else:
+            self.cos, self.sin = (F.embedding(positions, t) for t in tables)
         if ids is None:
             ids = torch.tensor(tokens, dtype=torch.int64).pin_memory().to(model.device, non_blocking=True)
         self.x = model.model.embed_tokens(ids).contiguous()
@@ -514,6 +559,14 @@ def _small_m(x, weight, bias):
     return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and m <= 16
             and n % 16 == 0 and k % 2048 == 0 and x.stride(1) == 1 and weight.is_contiguous()
             and (bias is None or bias.is_contiguous()))
+
+
+def _rope_rows(cfg, positions, dtype):
+    """cos and sin [len(positions), head_dim / 2] in `dtype`."""
+    D = cfg.head_dim
+    inv_freq = cfg.rope_theta ** (-torch.arange(0, D, 2, device=positions.device).float() / D)
+    angle = positions.float()[:, None] * inv_freq[None, :]
+    return angle.cos().to(dtype).contiguous(), angle.sin().to(dtype).contiguous()
 
 
 def _plain_norms(layer, dtype):

@@ -140,3 +140,21 @@ def test_rope_at_the_edges_of_its_chunks(gpu, dtype, rows, heads, D, extra, offs
     rk.rope_(t, heads, D, cos, sin)
     assert torch.equal(t[:, : heads * D].reshape(rows, heads, D), want)
     assert torch.equal(t[:, heads * D:], tail)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rope_tables_hold_the_rows_that_a_step_would_compute(monkeypatch, dtype):
+    from nano_hisparse import model as model_module
+
+    monkeypatch.setattr(model_module, "ROPE_TABLE_ROWS", 9000)
+    model = Model(ModelConfig(hidden_size=64, num_attention_heads=4, num_key_value_heads=2, num_hidden_layers=1)).to(dtype)
+    short = model._rope_tables(100)
+    assert len(short[0]) == 4096 and model._rope_tables(4096)[0] is short[0]
+    long = model._rope_tables(4097)
+    assert len(long[0]) == 8192 and model._rope_tables(5)[0] is long[0]
+    assert len(model._rope_tables(8500)[0]) == 9000 and model._rope_tables(9001) is None
+    positions = torch.tensor([0, 1, 4095, 4096, 8191])
+    for table, rows in zip(long, model_module._rope_rows(model.config, positions, dtype)):
+        assert torch.equal(F.embedding(positions, table), rows)
+    other = {torch.float32: torch.bfloat16}.get(dtype, torch.float32)
+    assert model.to(other)._rope_tables(10)[0].dtype == other  # tables of another dtype are made anew
