@@ -13,6 +13,7 @@ reused. The store knows no residency policy: callers place pages.
 from __future__ import annotations
 
 import contextlib
+import gc
 
 from collections import Counter
 from contextlib import nullcontext
@@ -234,12 +235,18 @@ class HostStore:
     def capturing(self, stream):
         """Within: cache operations may also run on `stream`, whose launches
         are being captured into a graph that is replayed on the compute
-        stream (so the stream order of cache work is unchanged)."""
+        stream (so the stream order of cache work is unchanged). Cyclic
+        garbage is left alone meanwhile: a dead cache is part of a cycle, and
+        its collection synchronises its streams, which fails the capture."""
         previous, self._capture_stream = self._capture_stream, stream
+        collects = gc.isenabled()
+        gc.disable()
         try:
             yield
         finally:
             self._capture_stream = previous
+            if collects:
+                gc.enable()
 
     def synchronize(self):
         if self.cuda:

@@ -354,3 +354,61 @@ def test_first_graph_step_fuses_the_projections_outside_the_capture(gpu, monkeyp
     engine.add_request("r", list(range(1, 20)), 4)
     engine.run()
     assert capturing and not any(capturing)
+
+
+def test_no_cyclic_garbage_is_collected_while_capturing():
+    import gc
+
+    storage = make_cache("cpu").storage
+    assert gc.isenabled()
+    with pytest.raises(KeyError):
+        with storage.capturing(None):
+            assert not gc.isenabled()
+            raise KeyError
+    assert gc.isenabled()
+    gc.disable()
+    try:
+        with storage.capturing(None):
+            pass
+        assert not gc.isenabled()  # a caller that keeps it off finds it off
+    finally:
+        gc.enable()
+
+
+@pytest.mark.gpu
+def test_a_cache_that_dies_during_a_capture_is_collected_after_it(gpu, monkeypatch):
+    """A cache is part of a reference cycle and synchronises its streams when
+    it is collected: collected inside a capture, it would fail the capture."""
+    import gc
+    import weakref
+
+    log_case(test="dead-cache-in-capture")
+    cfg = ModelConfig(vocab_size=64, hidden_size=2048, intermediate_size=2048, num_hidden_layers=1,
+                      num_attention_heads=16, num_key_value_heads=4)
+    torch.manual_seed(5)
+    model = Model(cfg).eval().to(gpu, torch.bfloat16)
+    held = [make_cache(str(gpu))]
+    dead = weakref.ref(held[0])
+    run_groups, alive = Model._run_groups, []
+
+    def dropping(self, *a):
+        if torch.cuda.is_current_stream_capturing():
+            held.clear()
+            _ = [[] for _ in range(5000)]  # enough allocations for the collector to run
+            alive.append(dead() is not None)
+        return run_groups(self, *a)
+
+    monkeypatch.setattr(Model, "_run_groups", dropping)
+    kv = CacheConfig(gpu_pages=64, host_pages=64, page_size=4, kv_heads=4, head_dim=128, dtype=torch.bfloat16,
+                     device=str(gpu))
+    engine = Engine(model, HybridKVCache(kv, HotConfig(16, 16)), top_k=4, batch_decode=True, graph=True)
+    engine.add_request("r", list(range(1, 20)), 4)
+    thresholds = gc.get_threshold()
+    gc.set_threshold(100, 1, 1)
+    try:
+        engine.run()
+    finally:
+        gc.set_threshold(*thresholds)
+    assert alive and all(alive)
+    gc.collect()
+    assert dead() is None
