@@ -16,7 +16,9 @@
 //  2. per sorted entry: page/offset, source and resident tables (staged in
 //     LDS at entry when they fit), host row, valid / resident_hit /
 //     needs_hot.
-//  3. an LDS hash of the host rows that need the hot buffer.
+//  3. an LDS hash of the host rows that need the hot buffer; with the fused
+//     selection, whose wanted rows are the first rows of whole pages, of the
+//     host pages only (32 keys in place of 2048 at 32 pages of 64).
 //  4. one coalesced pass over tags: a tag found in the hash is a hot hit for
 //     that host row and marks its slot protected.
 //  5. victims = lru stably partitioned (unprotected first): the lru values
@@ -28,9 +30,9 @@
 //     in lru order, m = min(n_miss, |U|) and e = n_miss - m, the new lru is
 //     U[m:] ++ U[:m] ++ Pr[e:] ++ Pr[:e], a rotation of each part. n_miss is
 //     summed with the protected count before the pass.
-//  6. miss ranks by a block scan; assigned slot = victims[rank].
-//  7. physical rows (scattered back to input order), compact miss plan, tag
-//     writes for misses.
+//  6. assigned slot of a miss = victims[rank], its rank from the wave sums of
+//     the reduction before 5; physical rows (scattered back to input order),
+//     compact miss plan, tag writes for misses.
 #include "select_common.h"
 
 namespace nhs {
@@ -46,6 +48,9 @@ constexpr int kWaves = kResolveThreads / 64;
 constexpr int kRankGroup = 4;   // 1024-slot chunks ranked per barrier
 constexpr int kTableCache = 2048;  // page table entries staged in LDS at entry
 constexpr int kFusedWavePages = kWave * 16;      // pages the fused select ranks in one wave
+constexpr int kPageBits = 11;
+constexpr int kPageCap = 1 << kPageBits;  // slots of the fused selection's page hash, at most
+static_assert(kPageCap >= 2 * kFusedWavePages, "load factor <= 1/2");
 constexpr int kFusedMaxPages = 4 * kFusedWavePages;  // ... in four waves (at most kWavesMaxTop chosen)
 
 struct ResolveArgs {
@@ -84,13 +89,17 @@ struct ResolveArgs {
   int32_t* positions_out;  // [batch, n]
 };
 
+// LDS of resolve_rows_kernel. Given positions: the phases' arrays share one
+// block, 92 KB. Fused selection: the page hash is small enough to lie beside
+// the tables (133 KB; the LDS holds one workgroup either way), so it is
+// cleared at entry and no barrier parts it from the phases before and after.
+template <bool kFused>
 struct ResolveShared {
   union {
     struct {
       uint64_t keys[kMaxK];           // phase 1-2
       int32_t src[kTableCache];       // the item's page tables, when they fit
       int32_t res[kTableCache];
-      int32_t chosen[kFusedWavePages]; // fused selection: chosen pages, ascending, -1 padded
     } e;
     struct {
       int32_t hkey[kHashCap];  // phase 3-4: wanted host rows
@@ -100,10 +109,36 @@ struct ResolveShared {
   } u;
   uint32_t prot[kMaxH / 32];  // protected slot bits
   int32_t victims[kMaxK];     // victims[0 .. min(n, H)-1]
-  int32_t red[2][kWaves * 8];                    // one scratch row per block reduction
+  int32_t red[kWaves * 8];                       // scratch of the block sums (and of the fused ranking)
   int32_t wcount[2][kRankGroup][kWaves];         // per-wave unprotected counts, double-buffered
   int32_t hot[kHotCache];                      // the item's hot block table, when it fits
 };
+template <>
+struct ResolveShared<true> {
+  struct {
+    union {
+      struct {
+        uint32_t cand[8 * kWavesMaxTop];  // phase 0: four_wave_rank's candidates
+        int32_t src[kTableCache];         // phases 0-2: the item's page tables, when they fit
+        int32_t res[kTableCache];
+        int32_t chosen[kFusedWavePages];  // phases 0-2: chosen pages, ascending, -1 padded
+      } e;
+      uint16_t lru16[kMaxH];  // phase 5
+    };
+    struct {
+      int32_t key[kPageCap];   // wanted host pages
+      int32_t at[kPageCap];    // a chosen page (its index in `chosen`) held there
+      int32_t rows[kPageCap];  // rows of it that are wanted, from its first
+      int32_t slot[kMaxK];     // hot slot holding entry j's host row, or -1
+    } pages;
+  } u;
+  uint32_t prot[kMaxH / 32];
+  int32_t victims[kMaxK];
+  int32_t red[kWaves * 8];
+  int32_t wcount[2][kRankGroup][kWaves];
+  int32_t hot[kHotCache];
+};
+static_assert(sizeof(ResolveShared<true>) <= 160 * 1024, "one workgroup's LDS");
 
 // Block reductions with one barrier each. Every call site passes its own
 // scratch row, so no barrier is needed before the scratch is reused.
@@ -114,6 +149,15 @@ __device__ __forceinline__ int row_sum(int x) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
   x += __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, false);  // row_half_mirror
   x += __builtin_amdgcn_update_dpp(0, x, 0x140, 0xF, 0xF, false);  // row_mirror
+  return x;
+}
+
+// Inclusive prefix sums over each 16-lane row of the wave.
+__device__ __forceinline__ int row_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
   return x;
 }
 
@@ -208,12 +252,8 @@ __device__ __forceinline__ void partition_lru(const uint16_t* lru16, const uint3
 #pragma unroll
     for (int c = 0; c < kRankGroup; ++c) {
       if (c < chunks) {
-        // inclusive scan of the wave counts over lanes 0..15 (row_shr 1, 2, 4, 8)
-        int x = lane < kWaves ? ucount[parity][c][lane] : 0;
-        x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);
-        x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
-        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
-        x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+        // inclusive scan of the wave counts over lanes 0..15
+        const int x = row_scan(lane < kWaves ? ucount[parity][c][lane] : 0);
         const int total_u = __builtin_amdgcn_readlane(x, kWaves - 1);
         const int waves_below = wave > 0 ? __builtin_amdgcn_readlane(x, wave - 1) : 0;
         const int n_valid = min(kResolveThreads, H - (g0 + c) * kResolveThreads);
@@ -288,15 +328,14 @@ __device__ __forceinline__ int hash_find(const int32_t* hkey, int32_t key) {
 template <int KPL, int KPL2 = 0>
 __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveArgs a) {
   constexpr int kSelectors = KPL == 0 ? 0 : KPL2 > 0 ? 4 : 1;  // waves that rank the scores
-  __shared__ ResolveShared sh;
+  constexpr bool kFused = KPL > 0;
+  __shared__ ResolveShared<kFused> sh;
   const int tid = threadIdx.x;
   const int b = blockIdx.x;
   const int n = a.n;
   const int H = a.hot_rows;
   const int P = a.page_size;
   const int64_t length = a.lengths ? a.lengths[b] : a.length;
-  int kp = 1;
-  while (kp < n) kp <<= 1;
   // fused selection: the ranking waves' score loads go first
   float sv[KPL > 0 ? KPL : 1];
   if constexpr (KPL > 0)
@@ -342,17 +381,41 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
       sh.u.e.res[i] = resident[i];
     }
 
+  // page hash of the fused selection: 4 to 8 slots per chosen page (at least
+  // 2 above 512 pages), the product's top bits, linear probing
+  const int page_bits = min(34 - __clz(a.top_pages), kPageBits);
+  const uint32_t page_mask = kFused ? (1u << page_bits) - 1 : 0;
+  auto page_slot = [&](int32_t page) { return ((uint32_t)page * 2654435761u) >> (32 - page_bits); };
+  auto find_page = [&](int32_t page) {  // its slot, or -1
+    if constexpr (kFused) {
+      uint32_t h = page_slot(page);
+      while (true) {
+        const int32_t k = sh.u.pages.key[h];
+        if (k == page) return (int)h;
+        if (k == -1) return -1;
+        h = (h + 1) & page_mask;
+      }
+    }
+    return -1;
+  };
+  if constexpr (kFused) {
+    for (int i = tid; i <= (int)page_mask; i += kResolveThreads) {
+      sh.u.pages.key[i] = sh.u.pages.at[i] = -1;
+      sh.u.pages.rows[i] = 0;
+    }
+    for (int i = tid; i < n; i += kResolveThreads) sh.u.pages.slot[i] = -1;
+    for (int i = tid; i < kMaxH / 32; i += kResolveThreads) sh.prot[i] = 0u;
+  }
+
   // ---- 0. fused selection --------------------------------------------------
   if constexpr (KPL > 0) {
     const int count = page_count(a.lengths, a.length, b, P, a.max_pages);
     if constexpr (KPL2 == 0) {
       if (tid < kWave) wave_rank<KPL>(sv, count, a.top_pages, a.mode, a.keep_sink, a.forced_key, sh.u.e.chosen);
     } else {
-      // the candidates live in the key array, unused until phase 1
-      static_assert(sizeof(sh.u.e.keys) >= 8 * 4 * kWavesMaxTop, "candidates fit the key array");
-      uint32_t* cand = reinterpret_cast<uint32_t*>(sh.u.e.keys);
+      uint32_t* cand = sh.u.e.cand;
       four_wave_rank<KPL, KPL2>(sv, count, a.top_pages, a.mode, a.keep_sink, a.forced_key, cand,
-                                reinterpret_cast<int32_t*>(cand + 4 * kWavesMaxTop), sh.red[0], sh.u.e.chosen);
+                                reinterpret_cast<int32_t*>(cand + 4 * kWavesMaxTop), sh.red, sh.u.e.chosen);
     }
     __syncthreads();
     for (int i = tid; i < a.top_pages; i += kResolveThreads) a.pages_out[(int64_t)b * a.top_pages + i] = sh.u.e.chosen[i];
@@ -364,9 +427,10 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
   // the end maps to `length`), so the page table lookups for the entries in
   // input order are issued right away (after the barrier, from LDS, when the
   // tables are staged) and kept when no pair is inverted. The fused
-  // selection's positions are in order by construction: pages ascending,
-  // and only the last page (count - 1, the highest chosen) or the padding
-  // pages hold positions at or past the length.
+  // selection's positions need no sort and no keys: they are in order and
+  // differ by construction (pages ascending, and only the last page, the
+  // highest chosen, or the padding pages hold positions at or past the
+  // length), and the barrier above has the tables staged.
   const int per = (n + kResolveThreads - 1) / kResolveThreads;  // <= kKPerThread
   const int j0 = tid * per;
   uint64_t key[kKPerThread];
@@ -380,65 +444,93 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
     src[q] = staged ? sh.u.e.src[page] : source[page];
     res[q] = staged ? sh.u.e.res[page] : resident[page];
   };
-#pragma unroll
-  for (int q = 0; q < kKPerThread; ++q) {
-    const int j = j0 + q;
-    key[q] = ~0ull;
-    src[q] = res[q] = -1;
-    if (q < per && j < n) {
-      int64_t raw;
-      if constexpr (KPL > 0) {
-        const uint32_t jp = a.page_div.div((uint32_t)j);
-        const int32_t p = sh.u.e.chosen[jp];
-        const int64_t t = (int64_t)p * P + (int64_t)((uint32_t)j - jp * (uint32_t)P);
-        raw = (p >= 0 && t < length) ? t : -1;
-        a.positions_out[(int64_t)b * n + j] = (int32_t)raw;
-      } else {
-        raw = a.positions_i64 ? static_cast<const int64_t*>(a.positions)[(int64_t)b * a.positions_stride + j]
-                              : (int64_t) static_cast<const int32_t*>(a.positions)[(int64_t)b * a.positions_stride + j];
-      }
-      const int64_t norm = (raw >= 0 && raw < length) ? raw : length;
-      key[q] = ((uint64_t)norm << 32) | (uint32_t)j;
-      sh.u.e.keys[j] = key[q];
-      if (!staged) lookup(q);
-    }
-  }
-  for (int i = n + tid; i < kp; i += kResolveThreads) sh.u.e.keys[i] = ~0ull;  // sort padding
-  __syncthreads();
-  bool sorted = true;
-  if constexpr (KPL == 0) {
-    int inverted = 0;
-    for (int i = tid; i + 1 < n; i += kResolveThreads) inverted |= sh.u.e.keys[i] > sh.u.e.keys[i + 1];
-    sorted = !__syncthreads_or(inverted);
-  }
-  if (sorted && staged) {
-#pragma unroll
-    for (int q = 0; q < kKPerThread; ++q)
-      if (q < per && j0 + q < n) lookup(q);
-  }
-  if (!sorted) {
-    for (int k = 2; k <= kp; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = tid; i < kp; i += kResolveThreads) {
-          int ixj = i ^ j;
-          if (ixj > i) {
-            uint64_t x = sh.u.e.keys[i], y = sh.u.e.keys[ixj];
-            bool up = (i & k) == 0;
-            if ((x > y) == up) {
-              sh.u.e.keys[i] = y;
-              sh.u.e.keys[ixj] = x;
-            }
-          }
+  if constexpr (kFused) {
+    // chosen page tid: its host page and wanted rows, if it needs the hot buffer
+    const int32_t p = tid < a.top_pages ? sh.u.e.chosen[tid] : -1;
+    const int64_t left = length - (int64_t)p * P;
+    if (p >= 0 && left > 0 && n_pages >= 1) {
+      const int page = min(p, n_pages - 1);
+      const int32_t host_page = staged ? sh.u.e.src[page] : source[page];
+      const int32_t res_page = staged ? sh.u.e.res[page] : resident[page];
+      if (host_page >= 0 && res_page < 0) {
+        uint32_t h = page_slot(host_page);
+        while (true) {
+          const int32_t prev = atomicCAS(&sh.u.pages.key[h], -1, host_page);
+          if (prev == -1 || prev == host_page) break;
+          h = (h + 1) & page_mask;
         }
-        __syncthreads();
+        // logical pages that share a host page settle on one entry, and the longer
+        atomicMax(&sh.u.pages.at[h], tid);
+        atomicMax(&sh.u.pages.rows[h], left < P ? (int32_t)left : P);
       }
     }
 #pragma unroll
     for (int q = 0; q < kKPerThread; ++q) {
       const int j = j0 + q;
+      key[q] = ~0ull;
+      src[q] = res[q] = -1;
       if (q < per && j < n) {
-        key[q] = sh.u.e.keys[j];
+        const uint32_t jp = a.page_div.div((uint32_t)j);
+        const int32_t p = sh.u.e.chosen[jp];
+        const int64_t t = (int64_t)p * P + (int64_t)((uint32_t)j - jp * (uint32_t)P);
+        const bool in = p >= 0 && t < length;
+        a.positions_out[(int64_t)b * n + j] = in ? (int32_t)t : -1;
+        key[q] = ((uint64_t)(in ? t : length) << 32) | (uint32_t)j;
         lookup(q);
+      }
+    }
+  } else {
+    int kp = 1;
+    while (kp < n) kp <<= 1;
+#pragma unroll
+    for (int q = 0; q < kKPerThread; ++q) {
+      const int j = j0 + q;
+      key[q] = ~0ull;
+      src[q] = res[q] = -1;
+      if (q < per && j < n) {
+        const int64_t raw =
+            a.positions_i64 ? static_cast<const int64_t*>(a.positions)[(int64_t)b * a.positions_stride + j]
+                            : (int64_t) static_cast<const int32_t*>(a.positions)[(int64_t)b * a.positions_stride + j];
+        const int64_t norm = (raw >= 0 && raw < length) ? raw : length;
+        key[q] = ((uint64_t)norm << 32) | (uint32_t)j;
+        sh.u.e.keys[j] = key[q];
+        if (!staged) lookup(q);
+      }
+    }
+    for (int i = n + tid; i < kp; i += kResolveThreads) sh.u.e.keys[i] = ~0ull;  // sort padding
+    __syncthreads();
+    int inverted = 0;
+    for (int i = tid; i + 1 < n; i += kResolveThreads) inverted |= sh.u.e.keys[i] > sh.u.e.keys[i + 1];
+    const bool sorted = !__syncthreads_or(inverted);
+    if (sorted && staged) {
+#pragma unroll
+      for (int q = 0; q < kKPerThread; ++q)
+        if (q < per && j0 + q < n) lookup(q);
+    }
+    if (!sorted) {
+      for (int k = 2; k <= kp; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          for (int i = tid; i < kp; i += kResolveThreads) {
+            int ixj = i ^ j;
+            if (ixj > i) {
+              uint64_t x = sh.u.e.keys[i], y = sh.u.e.keys[ixj];
+              bool up = (i & k) == 0;
+              if ((x > y) == up) {
+                sh.u.e.keys[i] = y;
+                sh.u.e.keys[ixj] = x;
+              }
+            }
+          }
+          __syncthreads();
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kKPerThread; ++q) {
+        const int j = j0 + q;
+        if (q < per && j < n) {
+          key[q] = sh.u.e.keys[j];
+          lookup(q);
+        }
       }
     }
   }
@@ -458,7 +550,10 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
     if (q < per && j < n) {
       int64_t lg = (int64_t)(key[q] >> 32);
       in_idx[q] = (int32_t)(key[q] & 0xffffffffu);
-      run_start[q] = j == 0 || (int64_t)(sh.u.e.keys[j - 1] >> 32) != lg;
+      if constexpr (kFused)
+        run_start[q] = lg < length;
+      else
+        run_start[q] = j == 0 || (int64_t)(sh.u.e.keys[j - 1] >> 32) != lg;
       bool unique = lg < length && run_start[q];
       uint32_t pg = a.page_div.div((uint32_t)lg);
       int32_t o = (int32_t)((uint32_t)lg - pg * (uint32_t)P);
@@ -470,36 +565,55 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
       res_blk[q] = (int32_t)res[q];
     }
   }
-  __syncthreads();  // keys are dead from here on; the union becomes the hash
+  __syncthreads();  // given positions: keys are dead from here on, the union becomes the hash; fused: pages hashed
 
   // ---- 3. hash of host rows that need the hot buffer -----------------------
-  for (int i = tid; i < kHashCap; i += kResolveThreads) {
-    sh.u.hash.hkey[i] = -1;
-    sh.u.hash.hslot[i] = -1;
-  }
-  for (int i = tid; i < kMaxH / 32; i += kResolveThreads) sh.prot[i] = 0u;
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < kKPerThread; ++q) {
-    if (!nhot[q]) continue;
-    int32_t key = (int32_t)host[q];
-    uint32_t h = hash_row(key) & (kHashCap - 1);
-    while (true) {
-      int32_t prev = atomicCAS(&sh.u.hash.hkey[h], -1, key);
-      if (prev == -1 || prev == key) break;
-      h = (h + 1) & (kHashCap - 1);
+  // Fused selection: the pages were hashed above, and each wanted row has a
+  // place of its own in pages.slot. No row is inserted or probed for, and the
+  // row hash's 64 KB, two barriers and the entries' keys fall away. A serial
+  // chain of LDS passes bounds this kernel: nine phases of 0.4 to 3.8 us. With
+  // the miss ranks taken from the reduction (one more barrier less), the
+  // whole launch in a captured graph, before -> now, us: 64 items of 2048
+  // pages, 32 of 32 rows chosen 14.8 -> 13.4; 16 of 512, 32 of 64 chosen
+  // 14.8 -> 13.5; 4 of 2048, 64 of 64 chosen 26.3 -> 23.1; 16 of 64, 4 of 16
+  // chosen 8.5 -> 7.6.
+  if constexpr (!kFused) {
+    for (int i = tid; i < kHashCap; i += kResolveThreads) {
+      sh.u.hash.hkey[i] = -1;
+      sh.u.hash.hslot[i] = -1;
     }
+    for (int i = tid; i < kMaxH / 32; i += kResolveThreads) sh.prot[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kKPerThread; ++q) {
+      if (!nhot[q]) continue;
+      int32_t key = (int32_t)host[q];
+      uint32_t h = hash_row(key) & (kHashCap - 1);
+      while (true) {
+        int32_t prev = atomicCAS(&sh.u.hash.hkey[h], -1, key);
+        if (prev == -1 || prev == key) break;
+        h = (h + 1) & (kHashCap - 1);
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
 
   // ---- 4. scan tags: hot hits and protected slots ---------------------------
   auto scan_tag = [&](int s, int32_t t) {
     if (t >= 0) {
-      int h = hash_find(sh.u.hash.hkey, t);
-      if (h >= 0) {
-        sh.u.hash.hslot[h] = s;
-        atomicOr(&sh.prot[s >> 5], 1u << (s & 31));
+      bool found;
+      if constexpr (kFused) {
+        const uint32_t page = a.page_div.div((uint32_t)t);
+        const int h = find_page((int32_t)page);
+        const int row = t - (int)(page * (uint32_t)P);
+        found = h >= 0 && row < sh.u.pages.rows[h];
+        if (found) sh.u.pages.slot[sh.u.pages.at[h] * P + row] = s;
+      } else {
+        const int h = hash_find(sh.u.hash.hkey, t);
+        found = h >= 0;
+        if (found) sh.u.hash.hslot[h] = s;
       }
+      if (found) atomicOr(&sh.prot[s >> 5], 1u << (s & 31));
     }
   };
 #pragma unroll
@@ -517,8 +631,11 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
     slot[q] = 0;
     local_rhit += rhit[q];
     if (nhot[q]) {
-      int h = hash_find(sh.u.hash.hkey, (int32_t)host[q]);
-      int32_t es = sh.u.hash.hslot[h];
+      int32_t es;
+      if constexpr (kFused)
+        es = sh.u.pages.slot[sh.u.pages.at[find_page((int32_t)src[q])] * P + off[q]];
+      else
+        es = sh.u.hash.hslot[hash_find(sh.u.hash.hkey, (int32_t)host[q])];
       hhit[q] = es >= 0;
       miss[q] = !hhit[q];
       slot[q] = es;
@@ -528,7 +645,7 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
   }
 
   // ---- 5. victims: lru stably partitioned, unprotected slots first ---------
-  __syncthreads();  // the hash is dead; the union now stages the lru
+  if constexpr (!kFused) __syncthreads();  // the hash is dead; the union now stages the lru
   // the lru is a permutation of [0, H); values are clamped so bad input stays in bounds
 #pragma unroll
   for (int i = 0; i < kRegH; ++i) {
@@ -539,21 +656,30 @@ __global__ __launch_bounds__(kResolveThreads) void resolve_rows_kernel(ResolveAr
     const int64_t v = lru_in[r];
     sh.u.lru16[r] = (uint16_t)(v < 0 ? 0 : v >= H ? H - 1 : v);
   }
+  // misses before this thread's, in its wave
+  int miss_before = row_scan(local_miss);
+  {
+    const int r0 = __builtin_amdgcn_readlane(miss_before, 15), r1 = __builtin_amdgcn_readlane(miss_before, 31),
+              r2 = __builtin_amdgcn_readlane(miss_before, 47);
+    const int row = (tid & 63) >> 4;
+    miss_before += (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0) - local_miss;
+  }
   // protected slots, misses, resident hits, hot hits
   int tot4[4] = {0, local_miss, local_rhit, local_hhit};
   for (int i = tid; i < (H + 31) / 32; i += kResolveThreads) tot4[0] += __popc(sh.prot[i]);
-  block_sums<4>(tot4, sh.red[0]);  // barrier: lru16 staged
-  const int n_prot = tot4[0];
+  block_sums<4>(tot4, sh.red);  // barrier: lru16 staged
+  {  // and in the waves below: every wave left its sums in the scratch row
+    const int lane = tid & 63, wave = tid >> 6;
+    const int x = row_scan(lane < kWaves ? sh.red[lane * 4 + 1] : 0);
+    miss_before += wave > 0 ? __builtin_amdgcn_readlane(x, wave - 1) : 0;
+  }
+  const int n_prot = tot4[0], n_miss = tot4[1];
   const int vlimit = n < H ? n : H;
   if (tid == 0) write_counts(a, b, tot4[2], tot4[3], tot4[1]);
   partition_lru(sh.u.lru16, sh.prot, H, n_prot, tot4[1], vlimit, sh.victims, lru_out, sh.wcount);
   __syncthreads();  // victims complete
 
-  // ---- 6. miss ranks ----------------------------------------------------------
-  int n_miss;
-  const int miss_before = block_scan(local_miss, sh.red[1], &n_miss);
-
-  // ---- 7. physical rows, plan, tag writes, counts ----------------------------
+  // ---- 6. physical rows, plan, tag writes, counts ----------------------------
   int64_t* phys_out = a.physical + (int64_t)b * a.plan_stride;
   int64_t* mh = a.miss_host + (int64_t)b * a.plan_stride;
   int64_t* md = a.miss_device + (int64_t)b * a.plan_stride;

@@ -120,6 +120,55 @@ def test_fused_select_resolve_equals_select_then_resolve(gpu, mode, B, Hq, Hkv, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "P,n_pages,top,H,spread",
+    [
+        (64, 60, 32, 2304, 8192 // 64),  # 256 hash slots for 32 pages; host pages whose rows agree in 13 bits
+        (3, 900, 1024, 4000, 1),  # every page chosen and more asked for: the fullest page hash
+        (7, 40, 1, 64, 1),  # one chosen page
+        (4096, 4, 1, 4096, 1),  # one page of every entry the LDS holds
+    ],
+)
+def test_fused_page_hash_with_shared_host_pages(gpu, P, n_pages, top, H, spread):
+    """Host pages that several logical pages share, one of them the partial
+    last page, tables narrower than the scores, tags of neighbouring rows and
+    of rows past the length: equal to the two launches, bit for bit."""
+    log_case(test="select-resolve-shared", P=P, n_pages=n_pages, top=top, H=H)
+    B = 3
+    rng = np.random.default_rng(P + n_pages)
+    n_hot = -(-H // P)
+    source = np.stack([rng.permutation(2 * n_pages)[:n_pages] * spread for _ in range(B)]).astype(np.int32)
+    resident = np.full((B, n_pages), -1, np.int32)
+    resident[:, 1::5] = rng.integers(0, 50, size=resident[:, 1::5].shape)
+    source[1, n_pages // 2 :] = source[1, : n_pages - n_pages // 2]  # each host page twice
+    source[2, -1] = source[2, 0]  # the last page, partial, shares the first one's host page
+    resident[2, -1] = resident[2, 0] = -1
+    hot = np.stack([rng.permutation(n_hot + 5)[:n_hot] for _ in range(B)]).astype(np.int32)
+    lengths = torch.tensor([n_pages * P, n_pages * P - P // 2, (n_pages - 1) * P + 1], device=gpu)
+    tags, lru = np.full((B, H), -1, np.int32), np.stack([rng.permutation(H) for _ in range(B)]).astype(np.int64)
+    for b in range(B):
+        rows = np.unique(np.concatenate([s * P + np.arange(P) for s in source[b]]))
+        keep = rng.permutation(rows)[: min(H // 2, rows.size)]
+        tags[b, rng.permutation(H)[: keep.size]] = keep
+    g_src, g_res, g_hot = (torch.from_numpy(x).to(gpu) for x in (source, resident, hot))
+    g = torch.Generator().manual_seed(P)
+    lo = torch.randn(B, n_pages, 2, 64, generator=g).to(gpu, torch.bfloat16)
+    q = torch.randn(B, 4, 64, generator=g).to(gpu, torch.bfloat16)
+    for table in (n_pages, max(1, n_pages // 2)):  # the narrower one ends in a page that the rest share
+        src, res = g_src[:, :table].contiguous(), g_res[:, :table].contiguous()
+        state = [(torch.from_numpy(tags).to(gpu), torch.from_numpy(lru).to(gpu)) for _ in range(2)]
+        pages, positions, _ = rk.quest_batched(q, lo, lo + 1, lengths, P, top)
+        _, _, scores = rk.quest_batched(q, lo, lo + 1, lengths, P, top, select=False)
+        # one step: a host row that two pages miss gets two slots, and the
+        # resolver's tags are defined to hold a row once
+        want = rk.resolve_batched(positions, src, res, g_hot, *state[0], lengths, P)
+        got = rk.select_resolve_batched(scores, src, res, g_hot, *state[1], lengths, P, top)
+        for x, y in zip((pages, positions) + tuple(want), got):
+            assert torch.equal(x, y), table
+        assert torch.equal(state[0][0], state[1][0]) and torch.equal(state[0][1], state[1][1])
+
+
+@pytest.mark.gpu
 def test_fused_select_resolve_rejects_shapes_beyond_its_selection(gpu):
     log_case(test="select-resolve-limits")
     B, H, P = 1, 8192, 8
