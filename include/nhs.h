@@ -384,6 +384,18 @@ int nhs_rope(int32_t rows, int32_t heads, int32_t head_dim, int32_t dtype, void*
 int nhs_silu_mul(int32_t rows, int32_t inter, int32_t dtype, const void* gate_up, void* out, void* stream);
 
 /*
+ * nhs_decode_rows: what a decode step reads by index, in one launch: x[b] =
+ * embed[ids[b]], cos_out[b] = cos[positions[b]], sin_out[b] =
+ * sin[positions[b]] for b < batch (<= 65535), rows copied bit for bit. embed is
+ * [embed_rows, row_bytes], cos and sin are [table_rows, half_bytes]; rows are
+ * whole 16-byte chunks and every base is 16-byte aligned. Indices beyond
+ * their table read its first or last row.
+ */
+int nhs_decode_rows(int32_t batch, const int64_t* ids, const int64_t* positions, const void* embed,
+                    int64_t embed_rows, int32_t row_bytes, const void* cos, const void* sin, int64_t table_rows,
+                    int32_t half_bytes, void* x, void* cos_out, void* sin_out, void* stream);
+
+/*
  * Linear layer for up to 16 token rows (decode): y[m, n] = sum_k x[m, k] *
  * w[n, k] (+ bias[n]), bf16 or fp16 (dtype), fp32 accumulation, one
  * rounding. w is [n, k] row-major (torch Linear weight layout); n a multiple

@@ -707,6 +707,32 @@ def silu_mul(gate_up):
     return out
 
 
+def decode_rows(ids, positions, embed, cos, sin):
+    """(embed[ids], cos[positions], sin[positions]) in one launch, or None
+    where the tables' rows are not aligned 16-byte chunks. ids and positions
+    are int64 [batch] within their tables; embed [vocab, hidden], cos and sin
+    [rows, head_dim / 2]."""
+    device = _require_gpu("decode_rows", ids, positions, embed, cos, sin)
+    if ids.shape != positions.shape or ids.ndim != 1 or ids.dtype != torch.int64 or positions.dtype != torch.int64 \
+            or not ids.is_contiguous() or not positions.is_contiguous():
+        raise ValueError("decode_rows: ids and positions are contiguous int64 [batch]")
+    if embed.ndim != 2 or cos.ndim != 2 or cos.shape != sin.shape or cos.dtype != sin.dtype:
+        raise ValueError("decode_rows: embed [vocab, hidden], cos and sin [rows, head_dim / 2]")
+    row, half = embed.shape[1] * embed.element_size(), cos.shape[1] * cos.element_size()
+    if row % 16 or half % 16 or row == 0 or half == 0 or len(embed) == 0 or len(cos) == 0 or len(ids) > 65535 \
+            or not (embed.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()) \
+            or (embed.data_ptr() | cos.data_ptr() | sin.data_ptr()) % 16:
+        return None
+    B = len(ids)
+    x = torch.empty(B, embed.shape[1], dtype=embed.dtype, device=device)
+    out = [torch.empty(B, cos.shape[1], dtype=cos.dtype, device=device) for _ in range(2)]
+    lib = _hip.load()
+    status = lib.nhs_decode_rows(B, _ptr(ids), _ptr(positions), _ptr(embed), len(embed), row, _ptr(cos), _ptr(sin),
+                                 len(cos), half, _ptr(x), _ptr(out[0]), _ptr(out[1]), _stream(device))
+    _hip.check(status, "nhs_decode_rows")
+    return x, *out
+
+
 # ---- prefill attention ---------------------------------------------------------------------
 
 

@@ -87,6 +87,23 @@ def test_silu_mul_matches_torch(gpu, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+# the smallest rows, the edge of a workgroup (256 chunks of 16 bytes) and past it
+@pytest.mark.parametrize("B,hidden,half", [(1, 8, 8), (16, 2048, 64), (3, 1936, 64), (7, 4096, 64), (2, 4104, 8)])
+def test_decode_rows_reads_the_tables_bit_for_bit(gpu, dtype, B, hidden, half):
+    g = torch.Generator(device=gpu).manual_seed(B)
+    embed = torch.randn(50, hidden, generator=g, device=gpu).to(dtype)
+    cos, sin = (torch.randn(90, half, generator=g, device=gpu).to(dtype) for _ in range(2))
+    ids = torch.randint(0, 50, (B,), generator=g, device=gpu)
+    positions = torch.randint(0, 90, (B,), generator=g, device=gpu)
+    ids[-1], positions[-1] = 49, 89
+    x, c, s = rk.decode_rows(ids, positions, embed, cos, sin)
+    assert torch.equal(x, embed[ids]) and torch.equal(c, cos[positions]) and torch.equal(s, sin[positions])
+    assert rk.decode_rows(ids, positions, embed[:, :-1].contiguous(), cos, sin) is None  # no whole chunks
+    assert rk.decode_rows(ids, positions, embed, cos[:, :-1].contiguous(), sin[:, :-1].contiguous()) is None
+
+
+@pytest.mark.gpu
 # (2048, 16, 4): q/k/v and o take nhs_linear_small_m in bf16
 @pytest.mark.parametrize("hidden,heads,kv_heads", [(128, 8, 2), (2048, 16, 4)])
 @pytest.mark.parametrize("micro_batches", [1, 2])
