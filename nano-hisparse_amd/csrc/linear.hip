@@ -36,9 +36,10 @@ enum { kEpiPlain = 0, kEpiSiluMul = 1, kEpiRope = 2 };
 typedef __bf16 lin_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 lin_f16x8 __attribute__((ext_vector_type(8)));
 typedef float lin_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t lin_u4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
-__device__ __forceinline__ lin_f32x4 lin_mfma(uint4 a, uint4 b, lin_f32x4 c) {
+__device__ __forceinline__ lin_f32x4 lin_mfma(lin_u4 a, lin_u4 b, lin_f32x4 c) {
   if constexpr (T::dtype == NHS_BF16)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lin_bf16x8, a), __builtin_bit_cast(lin_bf16x8, b),
                                                   c, 0, 0, 0);
@@ -64,6 +65,10 @@ struct LinearArgs {
 };
 
 template <typename T>
+__device__ __forceinline__ float lin_widen(uint16_t bits) {
+  return T::dtype == NHS_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+}
+template <typename T>
 __device__ __forceinline__ float lin_round(float v) {
   return T::dtype == NHS_BF16 ? bf16_bits_to_f32(f32_to_bf16_bits(v)) : f16_bits_to_f32(f32_to_f16_bits(v));
 }
@@ -75,6 +80,11 @@ __device__ __forceinline__ float lin_round(float v) {
 // TB/s against ~5.6 TB/s for long row segments. The region is private to
 // the wave and LDS executes a wave's operations in order, so no barrier is
 // needed between the writes and the reads.
+// A window's loads are all issued before the first wait. When a load of x was
+// left behind the wait for the weights and the epilogue's operands behind the
+// merge, the launches of 8 rows took, before -> now (us, cold): 2048 x 2048
+// 5.7 -> 5.3, 4096 x 4096 10.2 -> 9.4, 6144 x 4096 14.9 -> 14.2, 4096 x 14336
+// 26.6 -> 25.1, gate/up 28672 x 4096 45.3 -> 44.5.
 constexpr int kLinWindow = 256;                       // k elements staged per window (512 bytes of a row)
 constexpr int kLinRowBytes = kLinWindow * 2 + 16;     // staged row pitch (padded)
 
@@ -92,9 +102,11 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
   const int row = lane & 15, kq = (lane >> 4) * 8;  // MFMA operand row and element offset
   const int slice = a.k / waves;                     // a multiple of kLinWindow
   const int k_begin = wave * slice;
-  // tokens past m read row 0 and are zeroed (no branch between load and use)
-  const bool live_tok = row < a.m;
-  const char* xp = a.x + ((int64_t)(live_tok ? row : 0) * a.ldx + k_begin + kq) * T::bytes;
+  // tokens past m read row 0 and are zeroed, by a mask: of a select the
+  // compiler makes a branch, and puts a load of x behind it, after the wait
+  // for the weights
+  const uint32_t live = row < a.m ? ~0u : 0u;
+  const char* xp = a.x + ((int64_t)(row < a.m ? row : 0) * a.ldx + k_begin + kq) * T::bytes;
   // load mapping: instruction j covers tile rows 2j, 2j + 1 (lanes 0-31, 32-63), 16 bytes per lane
   const int lrow = lane >> 5, lcol = (lane & 31) * 16;
   const char* wrow = a.w + ((int64_t)(n0 + lrow) * a.ldw + k_begin) * T::bytes + lcol;
@@ -103,29 +115,52 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
   lin_f32x4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = (lin_f32x4){0.f, 0.f, 0.f, 0.f};
+  constexpr int kTile = kWave * 4;  // partial tile floats per wave and row tile
+  // The epilogue's operands are loaded before the weights, so that no load
+  // is left after the merge: as raw bits (a conversion here would wait for
+  // them) and unconditionally (threads without an output read another's,
+  // absent operands a weight).
+  const int ep_t = (int)threadIdx.x & (EPI == kEpiPlain ? kTile - 1 : kTile / 2 - 1);
+  const int ep_tok = (ep_t >> 2) & 15, ep_row = (ep_t >> 6) * 4 + (ep_t & 3);
+  const auto* ep_bias = reinterpret_cast<const uint16_t*>(a.bias ? a.bias : a.w);
+  uint16_t bias_bits[EPI == kEpiPlain ? RT : 2], cos_bits = 0, sin_bits = 0;
+  bool rotates = false;
+  if constexpr (EPI == kEpiPlain) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) bias_bits[rt] = ep_bias[a.bias ? n0 + rt * 16 + ep_row : 0];
+  } else {
+    bias_bits[0] = ep_bias[a.bias ? n0 + ep_row : 0];
+    bias_bits[1] = ep_bias[a.bias ? n0 + a.half + ep_row : 0];
+  }
+  if constexpr (EPI == kEpiRope) {
+    rotates = (int)blockIdx.x < a.rope_tiles;
+    const int at = rotates ? min(ep_tok, a.m - 1) * a.cs_len + (int)(blockIdx.x % a.per) * 8 + ep_row : 0;
+    cos_bits = reinterpret_cast<const uint16_t*>(rotates ? a.cos : a.w)[at];
+    sin_bits = reinterpret_cast<const uint16_t*>(rotates ? a.sin : a.w)[at];
+  }
   constexpr int kLoads = RT * 8;  // 16 rows per tile, two per instruction
   for (int w0 = 0; w0 < slice; w0 += kLinWindow) {
-    uint4 wv[kLoads], xv[kLinWindow / 32];
+    lin_u4 wv[kLoads], xv[kLinWindow / 32];
 #pragma unroll
     for (int j = 0; j < kLoads; ++j)
-      wv[j] = *reinterpret_cast<const uint4*>(wrow + ((int64_t)(2 * j) * a.ldw + (j >= 4 ? pair_skip : 0) + w0) * T::bytes);
+      wv[j] = *reinterpret_cast<const lin_u4*>(wrow + ((int64_t)(2 * j) * a.ldw + (j >= 4 ? pair_skip : 0) + w0) * T::bytes);
 #pragma unroll
     for (int s = 0; s < kLinWindow / 32; ++s)
-      xv[s] = *reinterpret_cast<const uint4*>(xp + (int64_t)(w0 + s * 32) * T::bytes);
+      xv[s] = *reinterpret_cast<const lin_u4*>(xp + (int64_t)(w0 + s * 32) * T::bytes);
+    __builtin_amdgcn_sched_barrier(0);  // all the window's loads are in flight before the first wait
 #pragma unroll
     for (int j = 0; j < kLoads; ++j)
-      *reinterpret_cast<uint4*>(stage + (2 * j + lrow) * kLinRowBytes + lcol) = wv[j];
+      *reinterpret_cast<lin_u4*>(stage + (2 * j + lrow) * kLinRowBytes + lcol) = wv[j];
 #pragma unroll
     for (int s = 0; s < kLinWindow / 32; ++s) {
-      const uint4 xb = live_tok ? xv[s] : make_uint4(0u, 0u, 0u, 0u);
+      const lin_u4 xb = xv[s] & live;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        const uint4 wa = *reinterpret_cast<const uint4*>(stage + (rt * 16 + row) * kLinRowBytes + (s * 32 + kq) * 2);
+        const lin_u4 wa = *reinterpret_cast<const lin_u4*>(stage + (rt * 16 + row) * kLinRowBytes + (s * 32 + kq) * 2);
         acc[rt] = lin_mfma<T>(wa, xb, acc[rt]);
       }
     }
   }
-  constexpr int kTile = kWave * 4;  // partial tile floats per wave and row tile
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
     *reinterpret_cast<float4*>(&red[(wave * RT + rt) * kTile + lane * 4]) =
@@ -136,10 +171,8 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
     // D lane l < 32 holds tile rows (l / 16) * 4 + i < 8; lane l + 32 holds
     // their partners 8 rows down, kTile / 2 floats further in each tile
     const int t = (int)threadIdx.x;
-    if (t >= kTile / 2) return;
-    const int l = t >> 2, i = t & 3, tok = l & 15;
-    if (tok >= a.m) return;
-    const int rho = (l >> 4) * 4 + i;
+    if (t >= kTile / 2 || ep_tok >= a.m) return;
+    const int tok = ep_tok, rho = ep_row;
     float lo = red[t], hi = red[t + kTile / 2];
     for (int w = 1; w < waves; ++w) {
       lo += red[w * kTile + t];
@@ -147,8 +180,8 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
     }
     const int n_lo = n0 + rho, n_hi = n0 + a.half + rho;
     if (a.bias) {
-      lo += load_elem(a.bias, T::dtype, n_lo);
-      hi += load_elem(a.bias, T::dtype, n_hi);
+      lo += lin_widen<T>(bias_bits[0]);
+      hi += lin_widen<T>(bias_bits[1]);
     }
     lo = lin_round<T>(lo);  // the projection's output, as the plain kernel stores it
     hi = lin_round<T>(hi);
@@ -157,10 +190,8 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
       store_elem(a.y, T::dtype, (int64_t)tok * a.ldy + (int64_t)blockIdx.x * 8 + rho, sg * hi);
     } else {
       float y_lo = lo, y_hi = hi;
-      if ((int)blockIdx.x < a.rope_tiles) {
-        const int d = (int)(blockIdx.x % a.per) * 8 + rho;
-        const float c = load_elem(a.cos, T::dtype, (int64_t)tok * a.cs_len + d);
-        const float sn = load_elem(a.sin, T::dtype, (int64_t)tok * a.cs_len + d);
+      if (rotates) {
+        const float c = lin_widen<T>(cos_bits), sn = lin_widen<T>(sin_bits);
         y_lo = lin_round<T>(lo * c) + lin_round<T>(-hi * sn);
         y_hi = lin_round<T>(hi * c) + lin_round<T>(lo * sn);
       }
@@ -170,16 +201,13 @@ __global__ __launch_bounds__(kLinMaxWaves * kWave) void linear_small_m_kernel(Li
     return;
   }
   // D lane l holds weight rows (l / 16) * 4 + i of the tile, token l % 16
-  for (int t = threadIdx.x; t < RT * kTile; t += (int)blockDim.x) {
-    const int rt = t / kTile, r = t - rt * kTile;
-    const int l = r >> 2, i = r & 3;
-    const int tok = l & 15;
-    if (tok >= a.m) continue;
-    float v = red[rt * kTile + r];
-    for (int w = 1; w < waves; ++w) v += red[(w * RT + rt) * kTile + r];
-    const int n = n0 + rt * 16 + (l >> 4) * 4 + i;
-    if (a.bias) v += load_elem(a.bias, T::dtype, n);
-    store_elem(a.y, T::dtype, (int64_t)tok * a.ldy + n, v);
+  if ((int)threadIdx.x >= kTile || ep_tok >= a.m) return;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    float v = red[rt * kTile + ep_t];
+    for (int w = 1; w < waves; ++w) v += red[(w * RT + rt) * kTile + ep_t];
+    if (a.bias) v += lin_widen<T>(bias_bits[rt]);
+    store_elem(a.y, T::dtype, (int64_t)ep_tok * a.ldy + n0 + rt * 16 + ep_row, v);
   }
 }
 
