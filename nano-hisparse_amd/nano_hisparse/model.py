@@ -370,7 +370,9 @@ class Model(nn.Module):
         """cos and sin [rows, head_dim / 2] in the model dtype of every
         position below `limit` (None beyond ROPE_TABLE_ROWS positions): kept
         with the model, longer ones (twice as long each) made on demand. A decode step
-        then reads its rows instead of computing them in eleven launches."""
+        then reads its rows instead of computing them in eleven launches.
+        Inside a graph capture, which cannot wait for a table, none is made
+        (None where no kept one is long enough)."""
         if limit > ROPE_TABLE_ROWS:
             return None
         cfg = self.config
@@ -379,12 +381,20 @@ class Model(nn.Module):
         for kept, tables in reversed(made):
             if kept == key and len(tables[0]) >= limit:
                 return tables
+        if self.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            return None
         rows = min(ROPE_TABLE_ROWS, max(4096, 1 << (limit - 1).bit_length()))
         tables = _rope_rows(cfg, torch.arange(rows, device=self.device), self.dtype)
         if self.device.type == "cuda":
             torch.cuda.current_stream(self.device).synchronize()  # complete for every stream from here on
         made.append((key, tables))
         return tables
+
+    def _span_tables(self, store, request_ids, spans):
+        """The cos/sin tables of each group's own positions (each by its
+        longest reservation: a group beyond ROPE_TABLE_ROWS has none, beside
+        another that does), for a capture that must make none."""
+        return [self._rope_tables(max(store.requests[r].max_tokens for r in request_ids[a:b])) for a, b in spans]
 
     def clear_decode_graphs(self):
         """Drops every captured decode-step graph, with the cache, buffers and
@@ -442,10 +452,9 @@ class Model(nn.Module):
             # Fuse before the capture: a fusion inside it would be recorded and not run, and every replay would
             # read the separate weights, which fusing frees.
             self._fused_projections()
-            # The same holds for cos/sin tables made inside it, and a workspace made inside it would be cleared by
-            # every replay.
-            limit = max(cache.storage.requests[r].max_tokens for r in request_ids)
-            tables = self._rope_tables(limit)
+            # The same holds for each group's cos/sin tables, and a workspace made inside it would be cleared by every
+            # replay.
+            tables = self._span_tables(store, request_ids, spans)
             buffers = [(torch.empty(2, b - a, dtype=torch.int64, device=cache.device),
                         torch.empty(b - a, dtype=torch.int64, device=cache.device)) for a, b in spans]
             steps = open_steps(buffers)
@@ -457,8 +466,8 @@ class Model(nn.Module):
             if overlap:
                 side.wait_stream(store.transfer)
             with store.capturing(side), torch.cuda.graph(graph, stream=side):
-                groups = [_Group(self, None, request_ids[a:b], cache, overlap, step=step, ids=ids)
-                          for (a, b), step, (_, ids) in zip(spans, steps, buffers)]
+                groups = [_Group(self, None, request_ids[a:b], cache, overlap, step=step, ids=ids, tables=made)
+                          for (a, b), step, (_, ids), made in zip(spans, steps, buffers, tables)]
                 logits = self._run_groups(groups, top_k)
             for step in steps:
                 step.forget_capture_events()
@@ -487,14 +496,16 @@ class _Last(NamedTuple):
 
 class _Group:
     """One batch group of decode_batch: its residual stream, RoPE tables,
-    cache step and the gather handle in flight."""
+    cache step and the gather handle in flight. Within a capture the step,
+    its token ids and its tables (or None) are made before and handed in."""
 
-    def __init__(self, model, tokens, request_ids, cache, overlap, step=None, ids=None):
+    def __init__(self, model, tokens, request_ids, cache, overlap, step=None, ids=None, tables=None):
         cfg = model.config
         self.model, self.cfg = model, cfg
         self.step = cache.decode_batch(request_ids, overlap) if step is None else step
         positions = self.step.dev_lengths[0]  # already on the device
-        tables = model._rope_tables(self.step.max_tokens)
+        if step is None:
+            tables = model._rope_tables(self.step.max_tokens)
         if ids is None:
             ids = torch.tensor(tokens, dtype=torch.int64).pin_memory().to(model.device, non_blocking=True)
         embed = model.model.embed_tokens

@@ -412,3 +412,38 @@ def test_a_cache_that_dies_during_a_capture_is_collected_after_it(gpu, monkeypat
     assert alive and all(alive)
     gc.collect()
     assert dead() is None
+
+
+@pytest.mark.gpu
+def test_graph_groups_with_and_without_kept_rope_tables(gpu, monkeypatch):
+    """Two groups of a graph step, one of which is reserved beyond the longest
+    kept cos/sin tables and computes its rows: no table is asked for within
+    the capture, and the tokens are the eager step's."""
+    from nano_hisparse import model as model_module
+
+    log_case(test="graph-rope-tables")
+    monkeypatch.setattr(model_module, "ROPE_TABLE_ROWS", 64)
+    cfg = ModelConfig(vocab_size=64, hidden_size=2048, intermediate_size=2048, num_hidden_layers=1,
+                      num_attention_heads=16, num_key_value_heads=4)
+    torch.manual_seed(5)
+    model = Model(cfg).eval().to(gpu, torch.bfloat16)
+    ask, capturing = Model._rope_tables, []
+
+    def asked(self, limit):
+        capturing.append(torch.cuda.is_current_stream_capturing())
+        return ask(self, limit)
+
+    monkeypatch.setattr(Model, "_rope_tables", asked)
+    tokens = []
+    for graph in (True, False):  # the graph step comes first: no table is there yet
+        kv = CacheConfig(gpu_pages=128, host_pages=128, page_size=4, kv_heads=4, head_dim=128, dtype=torch.bfloat16,
+                         device=str(gpu))
+        engine = Engine(model, HybridKVCache(kv, HotConfig(16, 16)), top_k=4, batch_decode=True, graph=graph,
+                        micro_batches=2)
+        engine.add_request("long", [i % 64 for i in range(100)], 6)
+        engine.add_request("short", list(range(1, 20)), 6)
+        requests = list(engine.waiting)
+        engine.run()
+        tokens.append([r.generated for r in requests])
+    assert capturing and not any(capturing)
+    assert tokens[0] == tokens[1]

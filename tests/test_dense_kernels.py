@@ -175,3 +175,40 @@ def test_rope_tables_hold_the_rows_that_a_step_would_compute(monkeypatch, dtype)
         assert torch.equal(F.embedding(positions, table), rows)
     other = {torch.float32: torch.bfloat16}.get(dtype, torch.float32)
     assert model.to(other)._rope_tables(10)[0].dtype == other  # tables of another dtype are made anew
+
+
+def test_a_captured_groups_tables_are_made_before_it(monkeypatch):
+    """Each group of a graph step has tables by its own longest reservation
+    (none beyond ROPE_TABLE_ROWS, beside a group that has some), made before
+    the capture: a group that is handed its step asks for none."""
+    from types import SimpleNamespace
+
+    from nano_hisparse import model as model_module
+
+    monkeypatch.setattr(model_module, "ROPE_TABLE_ROWS", 64)
+    model = Model(ModelConfig(hidden_size=64, num_attention_heads=4, num_key_value_heads=2, num_hidden_layers=1))
+    lengths = {"long": 65, "short": 50, "shorter": 20}
+    store = SimpleNamespace(requests={r: SimpleNamespace(max_tokens=n) for r, n in lengths.items()})
+    long, short = model._span_tables(store, list(lengths), [(0, 1), (1, 3)])
+    assert long is None and len(short[0]) == 64
+
+    def refused(limit):
+        raise AssertionError("a table was asked for within the capture")
+
+    monkeypatch.setattr(model, "_rope_tables", refused)
+    monkeypatch.setattr(model_module, "_decode_rows", lambda *a: None)  # a GPU kernel
+    positions = torch.tensor([7, 41])
+    step = SimpleNamespace(dev_lengths=torch.stack((positions, positions + 1)), max_tokens=50)
+    groups = [model_module._Group(model, None, None, None, False, step=step, ids=torch.tensor([1, 2]), tables=t)
+              for t in (long, short)]
+    assert torch.equal(groups[0].cos, groups[1].cos) and torch.equal(groups[0].sin, groups[1].sin)
+
+
+def test_no_table_is_made_while_a_stream_is_captured(monkeypatch):
+    monkeypatch.setattr(Model, "device", property(lambda self: torch.device("cuda:0")))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    model = Model(ModelConfig(hidden_size=64, num_attention_heads=4, num_key_value_heads=2, num_hidden_layers=1))
+    assert model._rope_tables(10) is None and not model.__dict__["_rope"]
+    kept = (torch.empty(20, 8), torch.empty(20, 8))
+    model._rope.append(((model.device, model.dtype, model.config.rope_theta, 16), kept))
+    assert model._rope_tables(20) is kept and model._rope_tables(21) is None
