@@ -1,12 +1,12 @@
 // Native forms of the hottest launchers of row_kernels.py, as a CPython
-// module (_launch).
+// module (_launch), and held_state, a check that a decode step makes.
 //
 // A launcher called from Python costs more than its kernel at small sizes:
 // 7 to 16 us of attribute reads, checks, tensor allocations and a ctypes
 // call, against 2 to 8 us of kernel. Here the operands are checked and the
 // outputs allocated on at::Tensor, and the library is called directly.
 //
-// Each function takes a well-formed call only: it returns None, with nothing
+// Each launcher takes a well-formed call only: it returns None, with nothing
 // launched or changed, as soon as an operand is anything but what
 // row_kernels.py would accept as it stands, and the Python launcher then
 // handles the call (it raises, converts or allocates as it always did). A
@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <stdexcept>
+#include <vector>
 
 #include "nhs.h"
 
@@ -482,12 +483,56 @@ PyObject* append_page(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   return PyLong_FromLong(st);
 }
 
+// ---- parameters --------------------------------------------------------------------------------
+
+// The bytes that tell whether the dicts (of modules' parameters and child
+// modules) hold what they held: each dict's size, and of each value a tensor's
+// address, dtype, sizes and strides or, of any other object and of a tensor
+// without them, its identity. For checks made on every step.
+PyObject* held_state(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 1 || !PyList_CheckExact(a[0])) {
+    PyErr_SetString(PyExc_TypeError, "held_state takes a list of dicts");
+    return nullptr;
+  }
+  std::vector<int64_t> state;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); ++i) {
+    PyObject* dict = PyList_GET_ITEM(a[0], i);
+    if (!PyDict_Check(dict)) {
+      PyErr_SetString(PyExc_TypeError, "held_state takes a list of dicts");
+      return nullptr;
+    }
+    state.push_back(PyDict_Size(dict));
+    PyObject *key, *value;
+    Py_ssize_t at = 0;
+    while (PyDict_Next(dict, &at, &key, &value)) {
+      if (!PyObject_TypeCheck(value, reinterpret_cast<PyTypeObject*>(THPVariableClass))) {
+        state.push_back((int64_t)(uintptr_t)value);
+        continue;
+      }
+      const size_t before = state.size();
+      try {
+        const Tensor& t = THPVariable_Unpack(value);
+        state.push_back((int64_t)(uintptr_t)t.const_data_ptr());
+        state.push_back((int64_t)t.scalar_type() << 32 | t.dim());
+        for (int64_t s : t.sizes()) state.push_back(s);
+        for (int64_t s : t.strides()) state.push_back(s);
+      } catch (const std::exception&) {
+        state.resize(before);
+        state.push_back((int64_t)(uintptr_t)value);
+      }
+    }
+  }
+  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(state.data()),
+                                   (Py_ssize_t)(state.size() * sizeof(int64_t)));
+}
+
 #define NHS_METHOD(name) \
   { #name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr }
 PyMethodDef methods[] = {NHS_METHOD(linear_small_m), NHS_METHOD(linear_silu_mul),   NHS_METHOD(linear_rope),
                          NHS_METHOD(add_rmsnorm),    NHS_METHOD(attend_batched),    NHS_METHOD(prefill_attention),
                          NHS_METHOD(quest_batched),  NHS_METHOD(select_resolve_batched),
-                         NHS_METHOD(append_page),    {nullptr, nullptr, 0, nullptr}};
+                         NHS_METHOD(append_page),    NHS_METHOD(held_state),
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

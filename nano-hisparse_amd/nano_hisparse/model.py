@@ -261,23 +261,16 @@ class Model(nn.Module):
         dicts and the per-request path are unchanged); fusing again happens
         only if a parameter was replaced since (e.g. by .to())."""
         fused = getattr(self, "_fused", None)
-        if fused is not None and fused[0] == self._projection_pointers():
+        if fused is not None and fused[0].unchanged():
             return fused[1]
-        layers = []
+        layers, modules = [], [self.model.layers]
         for layer in self.model.layers:
             attn, mlp = layer.self_attn, layer.mlp
-            qkv = (attn.q_proj, attn.k_proj, attn.v_proj)
-            layers.append((_fuse(qkv, "weight"), _fuse(qkv, "bias"), _fuse((mlp.gate_proj, mlp.up_proj), "weight")))
-        self._fused = (self._projection_pointers(), layers)
+            qkv, gate_up = (attn.q_proj, attn.k_proj, attn.v_proj), (mlp.gate_proj, mlp.up_proj)
+            layers.append((_fuse(qkv, "weight"), _fuse(qkv, "bias"), _fuse(gate_up, "weight")))
+            modules += (layer, attn, mlp, *qkv, *gate_up)
+        self._fused = (_Held(modules), layers)
         return layers
-
-    def _projection_pointers(self):
-        out = []
-        for layer in self.model.layers:
-            attn, mlp = layer.self_attn, layer.mlp
-            for m in (attn.q_proj, attn.k_proj, attn.v_proj, mlp.gate_proj, mlp.up_proj):
-                out.append(m.weight.data_ptr())
-        return out
 
     @torch.inference_mode()
     def decode_batch(self, tokens: list[int], request_ids: list, cache, top_k: int, micro_batches: int = 1,
@@ -419,7 +412,9 @@ class Model(nn.Module):
         and the requests' reserved pages, so the replayed step is the eager
         one. A graph is reused only while the cache's device item tables of
         the groups are the same objects (they hold the pointers the graph
-        read); otherwise it is captured again."""
+        read) and the model's modules and parameters are those it read
+        (model.to() replaces them and frees the old ones); otherwise it is
+        captured again."""
         store = cache.storage
         store.check_stream()
         graphs = self.__dict__.setdefault("_decode_graphs", {})
@@ -432,7 +427,8 @@ class Model(nn.Module):
         key = (tuple(request_ids), top_k, len(spans))
         items = [cache._layer_items(request_ids[a:b]) for a, b in spans]
         entry = graphs.get(key)
-        if entry is not None and (entry["cache"] is not cache or any(x is not y for x, y in zip(entry["items"], items))):
+        if entry is not None and (entry["cache"] is not cache or not entry["read"].unchanged()
+                                  or any(x is not y for x, y in zip(entry["items"], items))):
             del graphs[key]
             entry = None
         token_ids = [torch.tensor(tokens[a:b], dtype=torch.int64).pin_memory() for a, b in spans]
@@ -472,8 +468,9 @@ class Model(nn.Module):
             for step in steps:
                 step.forget_capture_events()
             # what the graph reads outside its own memory lives as long as it does
-            entry = {"cache": cache, "items": items, "buffers": buffers, "graph": graph, "logits": logits,
-                     "stream": side, "tables": tables, "workspaces": [step.workspace for step in steps]}
+            entry = {"cache": cache, "read": _Held(self.modules()), "items": items, "buffers": buffers, "graph": graph,
+                     "logits": logits, "stream": side, "tables": tables,
+                     "workspaces": [step.workspace for step in steps]}
             graphs[key] = entry
             while len(graphs) > 8:  # the most recent compositions keep their graphs
                 del graphs[next(iter(graphs))]
@@ -485,6 +482,25 @@ class Model(nn.Module):
         for step in steps:
             step.end()
         return entry["logits"].clone()
+
+
+class _Held:
+    """The parameters and child modules that some modules hold at one time,
+    to tell later whether they hold the same ones at the same addresses."""
+
+    def __init__(self, modules):
+        modules = list(modules)
+        self.dicts = [d for m in modules for d in (m._parameters, m._buffers, m._modules) if d]
+        self.children = [c for m in modules for c in m._modules.values()]  # held: their identities stay their own
+        self.state = self._now()
+
+    def _now(self):
+        from . import row_kernels as rk
+
+        return (rk._launch or rk._load_launch()).held_state(self.dicts)
+
+    def unchanged(self):
+        return self._now() == self.state
 
 
 class _Last(NamedTuple):

@@ -447,3 +447,84 @@ def test_graph_groups_with_and_without_kept_rope_tables(gpu, monkeypatch):
         tokens.append([r.generated for r in requests])
     assert capturing and not any(capturing)
     assert tokens[0] == tokens[1]
+
+
+def test_replaced_parameters_and_modules_are_noticed():
+    """What a captured graph and the fused projections read is compared by
+    address and layout: a graph replayed on other parameters would read the
+    old ones' freed memory."""
+    from nano_hisparse.model import _Held
+
+    model = Model(ModelConfig(num_hidden_layers=2)).eval()
+    attn, mlp = model.model.layers[1].self_attn, model.model.layers[0].mlp
+    read, fused = _Held(model.modules()), model._fused_projections()
+    assert not read.unchanged()  # fusing made the projections views of the fused tensors
+    read = _Held(model.modules())
+    model.load_state_dict(model.state_dict())  # in place
+    assert read.unchanged() and model._fused_projections() is fused
+    model.lm_head.weight = torch.nn.Parameter(model.lm_head.weight.detach().clone())
+    assert not read.unchanged() and model._fused_projections() is fused  # not one of the fused
+
+    def changed(change, refuses=True):
+        read, fused = _Held(model.modules()), model._fused_projections()
+        assert read.unchanged()
+        change()
+        assert not read.unchanged()
+        again = model._fused_projections()
+        assert (again is not fused) == refuses
+        for layer, (qkv, bias, _) in zip(model.model.layers, again):
+            a = layer.self_attn
+            assert torch.equal(qkv, torch.cat((a.q_proj.weight, a.k_proj.weight, a.v_proj.weight)))
+            assert torch.equal(bias, torch.cat((a.q_proj.bias, a.k_proj.bias, a.v_proj.bias)))
+
+    new = {k: torch.randn_like(v) for k, v in model.state_dict().items()}
+    changed(lambda: model.to(torch.bfloat16))
+    changed(lambda: model.to(torch.float32))
+    changed(lambda: setattr(attn.k_proj, "bias", torch.nn.Parameter(torch.randn_like(attn.k_proj.bias))))
+    changed(lambda: setattr(attn.v_proj, "weight", torch.nn.Parameter(torch.randn_like(attn.v_proj.weight))))
+    changed(lambda: setattr(mlp, "up_proj", torch.nn.Linear(128, 256, bias=False)))
+    changed(lambda: setattr(mlp.gate_proj.weight, "data", torch.randn(256, 128)))
+    changed(lambda: setattr(attn.o_proj, "weight", torch.nn.Parameter(torch.randn(128, 128))), refuses=False)
+    changed(lambda: model.load_state_dict(new, assign=True))
+
+
+@pytest.mark.gpu
+def test_a_graph_is_captured_again_after_parameters_were_replaced(gpu):
+    """Replaced parameters: the step equals the eager one on the new weights,
+    and replays from then on."""
+    log_case(test="graph-new-weights")
+    cfg = ModelConfig(vocab_size=64, hidden_size=2048, intermediate_size=2048, num_hidden_layers=2,
+                      num_attention_heads=16, num_key_value_heads=4)
+    torch.manual_seed(5)
+    model = Model(cfg).eval().to(gpu, torch.bfloat16)
+    caches = []
+    for _ in range(2):
+        kv = CacheConfig(gpu_pages=64, host_pages=64, page_size=4, kv_heads=4, head_dim=128, dtype=torch.bfloat16,
+                         device=str(gpu))
+        cache = HybridKVCache(kv, HotConfig(16, 16))
+        cache.reserve("r", 40, 2)
+        model.prefill(list(range(20)), cache, "r")
+        caches.append(cache)
+
+    def step(token):
+        replayed, eager = (model.decode_batch([token], ["r"], c, 4, graph=g) for c, g in zip(caches, (True, False)))
+        assert torch.equal(replayed, eager), token
+        return replayed
+
+    def graph():
+        return next(iter(model.__dict__["_decode_graphs"].values()))["graph"]
+
+    step(1)
+    first = graph()
+    before = step(2)
+    assert graph() is first
+    with torch.no_grad():
+        model.load_state_dict({k: v * 1.5 for k, v in model.state_dict().items()}, assign=True)
+    after = step(2)
+    second = graph()
+    assert second is not first and not torch.equal(before, after)
+    step(3)
+    assert graph() is second
+    model.lm_head = torch.nn.Linear(2048, 64, bias=False, device=gpu, dtype=torch.bfloat16)
+    step(4)
+    assert graph() is not second
