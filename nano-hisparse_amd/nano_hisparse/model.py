@@ -11,6 +11,7 @@ state dicts load either way and a seeded random init draws the same weights.
 
 from __future__ import annotations
 
+import sys
 from dataclasses import dataclass
 from typing import NamedTuple
 
@@ -182,7 +183,9 @@ class Model(nn.Module):
         if flash:
             from . import row_kernels as rk
         x = self.model.embed_tokens(upload(tokens, torch.int64, self.device))
-        if flash and all(_plain_norms(layer, x.dtype) for layer in self.model.layers):
+        if flash and all(_plain_layer(layer, x.dtype) for layer in self.model.layers):
+            if not _plain(self.model.embed_tokens, nn.Embedding):
+                x = x.clone()  # a hook may hold the rows, which are updated in place
             return self._prefill_layers(x, cache, request_id)
         for index, layer in enumerate(self.model.layers):
             q, k, v = self._project(layer, x, 0)
@@ -223,8 +226,9 @@ class Model(nn.Module):
                 cache.write(request_id, index, k, v)
             o = attn.o_proj(rk.prefill_attention(q, k, v).reshape(n, -1)).contiguous()
             delta = layer.mlp(rk.add_rmsnorm(x, o, norm2.weight, _eps(norm2, cfg))).contiguous()
-        last = _Last(x[-1:], delta[-1:])
-        return _linear(self._final_norm([last]), self.lm_head.weight, self.lm_head.bias)[0].float()
+        if _plain_norm(self.model.norm, x.dtype) and _plain(self.lm_head, nn.Linear):
+            return self._head([_Last(x[-1:], delta[-1:])])[0]
+        return self.lm_head(self.model.norm(x[-1] + delta[-1])).float()
 
     @torch.inference_mode()
     def decode(self, token: int, request_id, cache, top_k=None, backend="auto", selector="quest"):
@@ -345,19 +349,22 @@ class Model(nn.Module):
                         b.pre(index + 1, layers[index + 1], fused[index + 1], top_k)
             finally:
                 rk.set_gather_workgroups(0)
-        return _linear(self._final_norm(groups), self.lm_head.weight, self.lm_head.bias).float()
+        return self._head(groups)
 
-    def _final_norm(self, groups):
-        """The last residual add and norm of every group's rows."""
+    def _head(self, groups):
+        """The last residual add, the final norm and the lm_head of every
+        group's rows: fused kernels in place of a plain norm and head, else
+        the modules themselves."""
         from . import row_kernels as rk
 
-        norm = self.model.norm
-        if norm.weight.dtype == self.dtype and norm.weight.is_contiguous():
-            rows = [rk.add_rmsnorm(g.x, g.delta, norm.weight, _eps(norm, self.config), write_back=False)
-                    for g in groups]
-        else:
-            rows = [norm(g.x + g.delta) for g in groups]
-        return rows[0] if len(rows) == 1 else torch.cat(rows)
+        norm, head = self.model.norm, self.lm_head
+        plain = _plain_norm(norm, self.dtype)
+        rows = [rk.add_rmsnorm(g.x, g.delta, norm.weight, _eps(norm, self.config), write_back=False) if plain
+                else g.x + g.delta for g in groups]
+        x = rows[0] if len(rows) == 1 else torch.cat(rows)
+        if not plain:
+            x = norm(x)
+        return (_linear(x, head.weight, head.bias) if _plain(head, nn.Linear) else head(x)).float()
 
     def _rope_tables(self, limit):
         """cos and sin [rows, head_dim / 2] in the model dtype of every
@@ -504,7 +511,7 @@ class _Held:
 
 
 class _Last(NamedTuple):
-    """A prompt's last row, as _final_norm takes a group."""
+    """A prompt's last row, as _head takes a group."""
 
     x: torch.Tensor
     delta: torch.Tensor
@@ -581,8 +588,7 @@ def _decode_rows(embed, ids, positions, tables):
     472 us against 492 with three torch lookups)."""
     from . import row_kernels as rk
 
-    if (tables is None or type(embed) is not nn.Embedding or embed.max_norm is not None or embed._forward_hooks
-            or embed._forward_pre_hooks):
+    if tables is None or not _plain(embed, nn.Embedding) or embed.max_norm is not None:
         return None
     return rk.decode_rows(ids, positions, embed.weight, *tables)
 
@@ -616,11 +622,31 @@ def _rope_rows(cfg, positions, dtype):
     return angle.cos().to(dtype).contiguous(), angle.sin().to(dtype).contiguous()
 
 
-def _plain_norms(layer, dtype):
-    """Whether the layer's norms are weights of the activations' dtype, as
-    nhs_add_rmsnorm takes them."""
-    return all(n.weight.dtype == dtype and n.weight.is_contiguous()
-               for n in (layer.input_layernorm, layer.post_attention_layernorm))
+def _plain(module, *kinds):
+    """Whether a call of `module` is the forward of one of the `kinds` and
+    nothing more, so that a kernel may compute it from the weights: no
+    subclass, no forward of the instance's own, no hook."""
+    hooks = torch.nn.modules.module
+    return (type(module) in kinds and "forward" not in vars(module)
+            and not (module._forward_hooks or module._forward_pre_hooks or hooks._global_forward_hooks
+                     or hooks._global_forward_pre_hooks))
+
+
+def _plain_norm(norm, dtype):
+    """Whether `norm` is an RMSNorm that nhs_add_rmsnorm computes: this
+    module's or Qwen2's (from_pretrained), its weight in the activations'
+    dtype."""
+    qwen2 = sys.modules.get("transformers.models.qwen2.modeling_qwen2")
+    kinds = (RMSNorm,) if qwen2 is None else (RMSNorm, qwen2.Qwen2RMSNorm)
+    return _plain(norm, *kinds) and norm.weight.dtype == dtype and norm.weight.is_contiguous()
+
+
+def _plain_layer(layer, dtype):
+    """Whether _prefill_layers computes a layer's prompt pass: plain norms,
+    and plain q and k projections, whose outputs it rotates in place."""
+    attn = layer.self_attn
+    return (_plain_norm(layer.input_layernorm, dtype) and _plain_norm(layer.post_attention_layernorm, dtype)
+            and _plain(attn.q_proj, nn.Linear) and _plain(attn.k_proj, nn.Linear))
 
 
 def _eps(norm, cfg):

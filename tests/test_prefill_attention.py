@@ -112,3 +112,176 @@ def test_prefill_attention_of_infinite_and_nan_scores(gpu):
         assert torch.equal(a.isnan(), b.isnan())
         assert (a - b)[~b.isnan()].abs().max().item() <= 1e-2
     assert out[10, 0].isnan().all() and out[200:, 0].isnan().all() and not out[:, 1].isnan().any()
+
+
+# ---- the prompt pass ------------------------------------------------------------------------
+
+
+def rms_norm(x, weight, eps):
+    xf = x.float()
+    return (xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + eps)).to(x.dtype) * weight
+
+
+@pytest.fixture(params=["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)])
+def prompt_device(request, monkeypatch):
+    """The device of a model whose prompt pass is the one of a GPU model: on
+    the CPU its kernels are their torch expressions."""
+    from nano_hisparse import model as model_module
+
+    if request.param != "cpu":
+        return request.getfixturevalue("gpu")
+
+    def add_rmsnorm(x, delta, weight, eps, write_back=True):
+        h = x if delta is None else x.add_(delta) if write_back else x + delta
+        return rms_norm(h, weight, eps)
+
+    def rope_(t, heads, head_dim, cos, sin):
+        view = t.view(len(t), heads, head_dim)
+        lo, hi = view.chunk(2, -1)
+        c, s = torch.cat((cos, cos), -1)[:, None], torch.cat((sin, sin), -1)[:, None]
+        view.copy_(view * c + torch.cat((-hi, lo), -1) * s)
+
+    monkeypatch.setattr(model_module.Model, "device", property(lambda self: torch.device("cuda:0")))
+    monkeypatch.setattr(model_module, "upload", lambda values, dtype, device: torch.tensor(values, dtype=dtype))
+    monkeypatch.setattr(rk, "add_rmsnorm", add_rmsnorm)
+    monkeypatch.setattr(rk, "rope_", rope_)
+    monkeypatch.setattr(rk, "prefill_attention", lambda q, k, v: reference(q, k, v).to(q.dtype))
+    return "cpu"
+
+
+def prompt_model(device, dtype, head_dim=64, layers=2, seed=3):
+    from nano_hisparse.model import Model, ModelConfig
+
+    torch.manual_seed(seed)
+    cfg = ModelConfig(hidden_size=4 * head_dim, intermediate_size=512, num_hidden_layers=layers,
+                      num_attention_heads=4, num_key_value_heads=2, vocab_size=128)
+    model = Model(cfg).eval()
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if "norm" in name:
+                p.copy_(1 + 0.2 * torch.randn_like(p))
+    return model.to(device, dtype)
+
+
+TOKENS = [(7 * i * i + 3 * i) % 128 for i in range(70)]
+
+
+@pytest.mark.parametrize("where", ["norm1", "norm2", "norm", "lm_head"])
+def test_prompt_pass_calls_the_modules_that_are_not_plain(prompt_device, where):
+    """Forward hooks on the norms and the head run, and a norm or head of
+    another kind computes what it defines."""
+    print("case:", dict(test="prompt-modules", device=str(prompt_device), where=where), flush=True)
+    dtype = torch.bfloat16
+    plain = prompt_model(prompt_device, dtype)
+    want = plain.prefill(TOKENS)
+
+    def replace(model, make):
+        layer = model.model.layers[1]
+        owner, name = {"norm1": (layer, "input_layernorm"), "norm2": (layer, "post_attention_layernorm"),
+                       "norm": (model.model, "norm"), "lm_head": (model, "lm_head")}[where]
+        setattr(owner, name, make(getattr(owner, name)))
+
+    class Scaled(torch.nn.Module):  # the module with another parametrisation of its weight, exact: 4 * (w / 4)
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+            with torch.no_grad():
+                inner.weight.div_(4)
+            self.eps, self.bias = getattr(inner, "eps", None), None
+
+        @property
+        def weight(self):
+            return self.inner.weight
+
+        def forward(self, x):
+            w = self.inner.weight * 4
+            return torch.nn.functional.linear(x, w) if self.eps is None else rms_norm(x, w, self.eps)
+
+    calls = []
+
+    def hooked(module):
+        module.register_forward_hook(lambda m, args, out: calls.append(out.shape))
+        return module
+
+    def hooked_first(module):
+        module.register_forward_pre_hook(lambda m, args: calls.append(args[0].shape))
+        return module
+
+    def own_forward(module):
+        forward = module.forward
+        module.forward = lambda x: calls.append(x.shape) or forward(x)
+        return module
+
+    for make in (hooked, hooked_first, own_forward):
+        calls.clear()
+        model = prompt_model(prompt_device, dtype)
+        replace(model, make)
+        got = model.prefill(TOKENS)
+        assert len(calls) == 1, make.__name__
+        assert (got - want).norm() <= 2e-2 * want.norm(), make.__name__
+    model = prompt_model(prompt_device, dtype)
+    replace(model, Scaled)
+    got = model.prefill(TOKENS)
+    assert (got - want).norm() <= 2e-2 * want.norm()
+
+
+def test_prompt_pass_leaves_what_hooks_hold(prompt_device):
+    """q, k and the embedded rows that a hook keeps are the modules' outputs,
+    not the rotated and accumulated rows."""
+    print("case:", dict(test="prompt-hooks", device=str(prompt_device)), flush=True)
+    model = prompt_model(prompt_device, torch.bfloat16)
+    want = model.prefill(TOKENS)
+    attn = model.model.layers[0].self_attn
+    for module in (model.model.embed_tokens, attn.q_proj, attn.k_proj):
+        held = []
+        hook = module.register_forward_hook(lambda m, args, out: held.append((args[0], out, out.clone())))
+        got = model.prefill(TOKENS)
+        hook.remove()
+        (_, out, copy), = held
+        assert torch.equal(out, copy)
+        assert (got - want).norm() <= 2e-2 * want.norm()
+
+
+def test_the_norms_of_both_model_sources_are_plain():
+    """Qwen2's own norm and layer (from_pretrained) take the fused prompt pass
+    as this package's do; a subclass does not."""
+    from nano_hisparse.model import RMSNorm, _plain, _plain_layer, _plain_norm
+
+    modeling = pytest.importorskip("transformers.models.qwen2.modeling_qwen2")
+    transformers = pytest.importorskip("transformers")
+    cfg = transformers.Qwen2Config(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1,
+                                   num_attention_heads=4, num_key_value_heads=2)
+    hf = transformers.Qwen2ForCausalLM(cfg).eval()
+    model = prompt_model("cpu", torch.float32, layers=1)
+    for m in (hf, model):
+        assert _plain_layer(m.model.layers[0], torch.float32) and _plain_norm(m.model.norm, torch.float32)
+        assert not _plain_norm(m.model.norm, torch.bfloat16)
+        assert _plain(m.lm_head, torch.nn.Linear) and _plain(m.model.embed_tokens, torch.nn.Embedding)
+
+    class Other(RMSNorm):
+        pass
+
+    assert not _plain_norm(Other(8, 1e-6), torch.float32) and _plain_norm(RMSNorm(8, 1e-6), torch.float32)
+    assert isinstance(hf.model.norm, modeling.Qwen2RMSNorm)
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not _plain_norm(model.model.norm, torch.float32)
+    handle.remove()
+
+
+def test_the_batched_steps_head_calls_modules_that_are_not_plain():
+    """The decode step's last norm and lm_head (of one group and of two): a
+    hooked norm sees every row once, a hooked head too."""
+    from nano_hisparse.model import _Last
+
+    model = prompt_model("cpu", torch.float32, layers=1)
+    x, delta = torch.randn(5, 256), torch.randn(5, 256)
+    want = torch.nn.functional.linear(rms_norm(x + delta, model.model.norm.weight, 1e-6), model.lm_head.weight)
+    seen = []
+    model.model.norm.register_forward_hook(lambda m, args, out: seen.append(("norm", out.shape)))
+    model.lm_head.register_forward_hook(lambda m, args, out: seen.append(("lm_head", out.shape)))
+    for cuts in ([0, 5], [0, 3, 5]):
+        seen.clear()
+        with torch.inference_mode():
+            got = model._head([_Last(x[a:b], delta[a:b]) for a, b in zip(cuts, cuts[1:])])
+        assert seen == [("norm", (5, 256)), ("lm_head", (5, 128))]
+        torch.testing.assert_close(got, want)
