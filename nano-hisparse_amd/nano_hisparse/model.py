@@ -183,7 +183,8 @@ class Model(nn.Module):
         if flash:
             from . import row_kernels as rk
         x = self.model.embed_tokens(upload(tokens, torch.int64, self.device))
-        if flash and all(_plain_layer(layer, x.dtype) for layer in self.model.layers):
+        layers = self.model.layers
+        if flash and len(layers) and all(_plain_layer(layer, x.dtype) for layer in layers):
             if not _plain(self.model.embed_tokens, nn.Embedding):
                 x = x.clone()  # a hook may hold the rows, which are updated in place
             return self._prefill_layers(x, cache, request_id)

@@ -285,3 +285,12 @@ def test_the_batched_steps_head_calls_modules_that_are_not_plain():
             got = model._head([_Last(x[a:b], delta[a:b]) for a, b in zip(cuts, cuts[1:])])
         assert seen == [("norm", (5, 256)), ("lm_head", (5, 128))]
         torch.testing.assert_close(got, want)
+
+
+def test_prompt_pass_of_no_layers(prompt_device):
+    print("case:", dict(test="prompt-no-layers", device=str(prompt_device)), flush=True)
+    model = prompt_model(prompt_device, torch.bfloat16, layers=0)
+    with torch.inference_mode():
+        row = model.model.embed_tokens.weight[TOKENS[-1]]
+        want = torch.nn.functional.linear(rms_norm(row, model.model.norm.weight, 1e-6), model.lm_head.weight)
+    assert torch.equal(model.prefill(TOKENS), want.float())
