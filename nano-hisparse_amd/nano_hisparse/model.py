@@ -370,25 +370,30 @@ class Model(nn.Module):
     def _rope_tables(self, limit):
         """cos and sin [rows, head_dim / 2] in the model dtype of every
         position below `limit` (None beyond ROPE_TABLE_ROWS positions): kept
-        with the model, longer ones (twice as long each) made on demand. A decode step
-        then reads its rows instead of computing them in eleven launches.
-        Inside a graph capture, which cannot wait for a table, none is made
-        (None where no kept one is long enough)."""
+        with the model while its device, dtype and RoPE stay, longer ones
+        (twice as long each) made on demand. A decode step then reads its
+        rows instead of computing them in eleven launches. Inside a graph
+        capture, which cannot wait for a table, none is made (None where no
+        kept one is long enough)."""
         if limit > ROPE_TABLE_ROWS:
             return None
         cfg = self.config
         key = (self.device, self.dtype, cfg.rope_theta, cfg.head_dim)
-        made = self.__dict__.setdefault("_rope", [])  # every table made: other streams may still read the shorter ones
-        for kept, tables in reversed(made):
-            if kept == key and len(tables[0]) >= limit:
+        stream = torch.cuda.current_stream(self.device) if self.device.type == "cuda" else None
+        made = [entry for entry in self.__dict__.get("_rope", ()) if entry[0] == key]
+        for _, tables, home in reversed(made):
+            if len(tables[0]) >= limit:
+                if stream != home:
+                    for t in tables:
+                        t.record_stream(stream)
                 return tables
-        if self.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+        if stream is not None and torch.cuda.is_current_stream_capturing():
             return None
         rows = min(ROPE_TABLE_ROWS, max(4096, 1 << (limit - 1).bit_length()))
         tables = _rope_rows(cfg, torch.arange(rows, device=self.device), self.dtype)
-        if self.device.type == "cuda":
-            torch.cuda.current_stream(self.device).synchronize()  # complete for every stream from here on
-        made.append((key, tables))
+        if stream is not None:
+            stream.synchronize()  # complete for every stream from here on
+        self.__dict__["_rope"] = [*made, (key, tables, stream)]
         return tables
 
     def _span_tables(self, store, request_ids, spans):
@@ -399,8 +404,13 @@ class Model(nn.Module):
 
     def clear_decode_graphs(self):
         """Drops every captured decode-step graph, with the cache, buffers and
-        graph memory each one holds."""
+        graph memory each one holds, and the kept cos/sin tables."""
         self.__dict__.pop("_decode_graphs", None)
+        self.__dict__.pop("_rope", None)
+
+    def __getstate__(self):
+        # graphs, tables and fused projections stay with this object: a copy makes its own
+        return {k: v for k, v in self.__dict__.items() if k not in ("_decode_graphs", "_rope", "_fused")}
 
     def _decode_batch_graph(self, tokens, request_ids, cache, top_k, cuts):
         """decode_batch with the step's launches (every layer of every group,

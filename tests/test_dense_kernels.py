@@ -207,8 +207,37 @@ def test_a_captured_groups_tables_are_made_before_it(monkeypatch):
 def test_no_table_is_made_while_a_stream_is_captured(monkeypatch):
     monkeypatch.setattr(Model, "device", property(lambda self: torch.device("cuda:0")))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: "stream")
     model = Model(ModelConfig(hidden_size=64, num_attention_heads=4, num_key_value_heads=2, num_hidden_layers=1))
-    assert model._rope_tables(10) is None and not model.__dict__["_rope"]
+    assert model._rope_tables(10) is None and "_rope" not in model.__dict__
     kept = (torch.empty(20, 8), torch.empty(20, 8))
-    model._rope.append(((model.device, model.dtype, model.config.rope_theta, 16), kept))
+    model._rope = [((model.device, model.dtype, model.config.rope_theta, 16), kept, "stream")]
     assert model._rope_tables(20) is kept and model._rope_tables(21) is None
+
+
+def test_rope_tables_go_with_what_they_were_made_for():
+    """Tables of an earlier dtype are dropped when new ones are made,
+    clear_decode_graphs() drops all of them, and a copy of the model carries
+    none along."""
+    import copy
+    import io
+    import weakref
+
+    model = Model(ModelConfig(hidden_size=64, num_attention_heads=4, num_key_value_heads=2, num_hidden_layers=1))
+    old = [weakref.ref(model._rope_tables(n)[0]) for n in (10, 5000)]
+    assert len(model._rope) == 2
+    new = model.to(torch.bfloat16)._rope_tables(10)
+    assert len(model._rope) == 1 and model._rope_tables(10) is new and all(r() is None for r in old)
+    model._fused_projections()
+    buffer = io.BytesIO()
+    torch.save(model, buffer)
+    buffer.seek(0)
+    for other in (copy.deepcopy(model), torch.load(buffer, weights_only=False)):
+        assert not {"_rope", "_fused", "_decode_graphs"} & set(other.__dict__)
+        assert all(torch.equal(a, b) for a, b in zip(other.parameters(), model.parameters()))
+        qkv = other._fused_projections()[0][0]
+        assert torch.equal(qkv, model._fused_projections()[0][0]) and qkv is not model._fused_projections()[0][0]
+    gone = weakref.ref(new[0])
+    model.clear_decode_graphs()
+    del new
+    assert gone() is None
