@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import contextlib
 import gc
+import threading
 
 from collections import Counter
 from contextlib import nullcontext
@@ -36,6 +37,30 @@ def upload(values, dtype, device):
     if torch.device(device).type != "cuda":
         return host.to(device)
     return host.pin_memory().to(device, non_blocking=True)
+
+
+_pauses = threading.Lock()
+_paused = [0, False]  # captures in progress, whether collection was on before the first
+
+
+@contextlib.contextmanager
+def _collection_paused():
+    """No cyclic garbage is collected within, however many captures overlap
+    (several threads): the last to end turns collection back on, if it was
+    on before the first."""
+    with _pauses:
+        if not _paused[0]:
+            _paused[1] = gc.isenabled()
+            gc.disable()
+        _paused[0] += 1
+    try:
+        yield
+    finally:
+        with _pauses:
+            _paused[0] -= 1
+            if not _paused[0] and _paused[1]:
+                gc.enable()
+
 
 PageKey = tuple  # (request_id, layer, page index)
 
@@ -239,14 +264,11 @@ class HostStore:
         garbage is left alone meanwhile: a dead cache is part of a cycle, and
         its collection synchronises its streams, which fails the capture."""
         previous, self._capture_stream = self._capture_stream, stream
-        collects = gc.isenabled()
-        gc.disable()
         try:
-            yield
+            with _collection_paused():
+                yield
         finally:
             self._capture_stream = previous
-            if collects:
-                gc.enable()
 
     def synchronize(self):
         if self.cuda:

@@ -528,3 +528,18 @@ def test_a_graph_is_captured_again_after_parameters_were_replaced(gpu):
     model.lm_head = torch.nn.Linear(2048, 64, bias=False, device=gpu, dtype=torch.bfloat16)
     step(4)
     assert graph() is not second
+
+
+def test_garbage_waits_for_every_overlapping_capture():
+    """Captures of two caches (two threads) that end in the order they began:
+    collection stays off until the second ends."""
+    import gc
+
+    first, second = (make_cache("cpu").storage.capturing(None) for _ in range(2))
+    assert gc.isenabled()
+    first.__enter__()
+    second.__enter__()
+    first.__exit__(None, None, None)
+    assert not gc.isenabled()
+    second.__exit__(None, None, None)
+    assert gc.isenabled()
