@@ -460,16 +460,19 @@ PyObject* select_resolve_batched(PyObject*, PyObject* const* a, Py_ssize_t nargs
 
 // ---- append ------------------------------------------------------------------------------------
 
-// nhs_append_page with the arguments row_kernels.PageAppender prepared (checked there), as whole numbers; returns the
-// status.
+// nhs_append_page with the arguments row_kernels.PageAppender prepared (checked there), as whole numbers of any integer
+// type; returns the status.
 PyObject* append_page(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (nargs != 17) {
     PyErr_SetString(PyExc_TypeError, "wrong number of arguments");
     return nullptr;
   }
   int64_t v[17];
-  for (int i = 0; i < 17; ++i) {
-    v[i] = (int64_t)PyLong_AsUnsignedLongLong(a[i]);
+  for (int i = 0; i < 17; ++i) {  // negative numbers go to the library, which refuses them
+    PyObject* whole = PyNumber_Index(a[i]);
+    if (!whole) return nullptr;
+    v[i] = (int64_t)PyLong_AsUnsignedLongLongMask(whole);
+    Py_DECREF(whole);
     if (PyErr_Occurred()) return nullptr;
   }
   const auto at = [&](int i) { return reinterpret_cast<void*>((uintptr_t)v[i]); };
