@@ -306,7 +306,8 @@ class Model(nn.Module):
         if micro_batches not in (1, 2):
             raise ValueError("micro_batches must be 1 or 2")
         n = len(tokens)
-        if n and not 0 <= min(tokens) <= max(tokens) < len(self.model.embed_tokens.weight):
+        embed = self.model.embed_tokens
+        if n and _plain(embed, nn.Embedding) and not 0 <= min(tokens) <= max(tokens) < len(embed.weight):
             raise IndexError("token id outside the vocabulary")
         if n < 2:
             micro_batches = 1

@@ -543,3 +543,20 @@ def test_garbage_waits_for_every_overlapping_capture():
     assert not gc.isenabled()
     second.__exit__(None, None, None)
     assert gc.isenabled()
+
+
+def test_token_ids_are_checked_for_a_plain_embedding_only():
+    """A plain embedding's rows are read by index, so ids beyond them are
+    refused; a module of another kind decides itself what its ids mean."""
+    class Wrapped(torch.nn.Embedding):
+        def forward(self, ids):
+            return super().forward(ids % self.num_embeddings)
+
+    cache = make_cache("cpu")
+    model = Model(ModelConfig(vocab_size=64)).eval()
+    for token in (64, -1):
+        with pytest.raises(IndexError, match="vocabulary"):
+            model.decode_batch([token], ["a"], cache, 2)
+    model.model.embed_tokens = Wrapped(64, 128)
+    with pytest.raises(RuntimeError, match="GPU cache"):  # past the check of the ids
+        model.decode_batch([64], ["a"], cache, 2)
