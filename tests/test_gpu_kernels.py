@@ -692,3 +692,29 @@ def test_append_rows_at_the_edges_of_passes_and_chunks(gpu, dtype, P, Hkv, D):
 ])
 def test_attend_rows_where_the_split_count_changes(gpu, dtype, Hq, Hkv, D, P, N):
     test_attend_rows_matches_oracle(gpu, dtype, dtype, 1, Hq, Hkv, D, P, N, False)
+
+
+@pytest.mark.gpu
+def test_attend_fp32_rounds_its_accumulators_once_per_row_group(gpu):
+    """fp32 attention over 4096 rows a workgroup (16 requests of 32/8 heads of
+    128: one split, 256 rows per lane slot in 64 groups) against float64. A
+    relative 2.2e-7 with one rounding of an accumulator per group of four
+    rows and the eight waves' sums added in pairs; 3.3e-7 with a rounding for
+    each row and each rescale. Half-way between is refused."""
+    log_case(test="attend-fp32-error")
+    g = torch.Generator(device=gpu).manual_seed(2)
+    B, Hq, Hkv, D, P, n = 16, 32, 8, 128, 64, 4096
+    pool = rk.padded_pool(B * n // P, P, Hkv, D, torch.float32, gpu)
+    pool.copy_(torch.randn(pool.shape, generator=g, device=gpu))
+    q = torch.randn(B, Hq, D, generator=g, device=gpu)
+    rows = torch.randperm(B * n, generator=g, device=gpu).view(B, n)
+    out = rk.attend_batched(q, pool, rows, P).double()
+    off = size = 0.0
+    for b in range(B):
+        kv = pool[rows[b] // P, :, rows[b] % P].double()
+        k, v = (x.repeat_interleave(Hq // Hkv, 1) for x in (kv[:, 0], kv[:, 1]))
+        p = torch.softmax((q[b].double() * k).sum(-1) * D**-0.5, 0)
+        want = (p[:, :, None] * v).sum(0)
+        off += (out[b] - want).square().sum().item()
+        size += want.square().sum().item()
+    assert (off / size) ** 0.5 <= 2.75e-7
