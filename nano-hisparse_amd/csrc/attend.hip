@@ -41,12 +41,16 @@ constexpr int kMinRowsPerSplit = 32;  // the workspace holds partials for splits
 // to split: a split costs the merge's store -> atomic -> load chain and every
 // further one lengthens the merge, while one workgroup reads several hundred
 // rows in a round trip or two. attend_kernel: four row groups of its eight
-// waves, at most kSplitRows. us at 32 rows per split / these, one request of
-// 4/2 heads of 64, fp32: 128 rows 8.8 / 5.2, 512 rows 16.2 / 7.0, 2048 rows
-// 25.6 / 10.6; 14/2 heads of 64, bf16, 2048 rows 35.1 / 15.2; 32/8 heads of
-// 128, fp32, 2048 rows 22.9 / 17.1 (half as many: 22.8; twice: 17.4).
-// attend_mfma_kernel (32/8 heads of 128, bf16, 128 rows per split / 256): 256
-// rows 9.4 / 7.3, 2048 rows 11.5 / 10.0 (512 rows per split: 12.0).
+// waves, at most kSplitRows. us at 32 rows per split / these, every launch on
+// rows untouched for 700 MB of other reads: one request of 4/2 heads of 64,
+// fp32: 128 rows 8.8 / 5.5, 512 rows 16.2 / 9.4, 2048 rows 25.5 / 13.0, and
+// eight of them 9.9 / 6.6, 13.1 / 9.8, 14.8 / 14.0; 14/2 heads of 64, bf16,
+// 2048 rows 35.2 / 16.2; 32/8 heads of 128, fp32: 512 rows 22.6 / 13.3 (four
+// requests 13.7 / 14.0, the most lost of 144 shapes), 2048 rows 24.2 / 18.7.
+// attend_mfma_kernel (128 rows per split / 256), 32/8 heads of 128, bf16: 256
+// rows 10.5 / 8.4, 2048 rows 12.5 / 11.2; 2 requests x 2048 rows 14.6 / 12.2,
+// 4 x 1024 12.8 / 11.8, 8 x 512 12.5 / 11.6, 8 x 256 11.2 / 8.8; 28/4 heads
+// of 128: 1 x 1024 13.6 / 13.9, 4 x 2048 18.0 / 15.1.
 constexpr int kSplitRows = 512;
 constexpr int kMSplitRows = 256;
 constexpr int kStage = 4096;  // row indices staged in LDS per pass (16 KiB)
