@@ -132,7 +132,7 @@ __device__ __forceinline__ std::conditional_t<T::bytes == 4, float, uint16_t> na
   else return T::dtype == NHS_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
 }
 
-// Chunk `index` of the new rows of one plane (rows one after another).
+// 16-byte chunk `chunk` of new row `row` of one plane.
 __device__ __forceinline__ const NHS_GLOBAL append_u4* new_chunk(const AppendArgs& a, int plane, uint32_t row,
                                                                  uint32_t chunk, int esize) {
   const NHS_GLOBAL char* src = to_global(static_cast<const char*>(plane ? a.v : a.k));
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kAppendThreads) void append_items_kernel(AppendItem
   append_element<T>(a, e);
 }
 
-// Whether rows are whole 16-byte chunks wherever append_rows touches them.
+// Whether rows are whole 16-byte chunks wherever append_page_rows_kernel touches them.
 static bool whole_chunks(const void* k, const void* v, const void* pool, const void* host, int64_t pool_block_stride,
                          int64_t token_stride, int64_t row_elems, int esize) {
   return row_elems * esize % 16 == 0 && token_stride * esize % 16 == 0 && pool_block_stride % 16 == 0 &&

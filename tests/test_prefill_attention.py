@@ -114,6 +114,53 @@ def test_prefill_attention_of_infinite_and_nan_scores(gpu):
     assert out[10, 0].isnan().all() and out[200:, 0].isnan().all() and not out[:, 1].isnan().any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(500, 2, 1, 64), (4001, 2, 1, 128), (3100, 32, 8, 128)])
+@pytest.mark.parametrize("dtype,subnormal", [(torch.float16, 16), (torch.float16, 22), (torch.bfloat16, 16)])
+def test_prefill_attention_of_one_dominating_key_and_many_small_ones(gpu, dtype, subnormal, S, Hq, Hkv, D):
+    """Weights of 2^-subnormal beside one of 1 (fp16: subnormal numbers) count
+    alike in the numerator (MFMA) and the denominator (packed dot products):
+    the values are 0 for the dominating key and 1 for the others, so an
+    output is S / (1 + S) with S the small weights' sum, and flushing them in
+    either sum alone would show as S or as S^2.
+
+    A weight is rounded to the dtype: by half a unit in the last place, 2^-25
+    at most for an fp16 weight below 2^-13 and 2^-8 of itself in bf16 (eight
+    significant bits). So S is off by at most n * 2^-25 or 2^-8 * S, and the
+    output by that and its own rounding, 2^-11 or 2^-8 of itself (plus one
+    subnormal unit, 2^-24)."""
+    print("case:", dict(S=S, Hq=Hq, Hkv=Hkv, D=D, dtype=str(dtype), subnormal=subnormal), flush=True)
+    q, k, v = (torch.zeros(S, h, D, device=gpu, dtype=dtype) for h in (Hq, Hkv, Hkv))
+    q[..., 0] = 8
+    k[0, :, 0] = subnormal * 0.6931471805599453 * D**0.5 / 8
+    v[1:] = 1
+    out = rk.prefill_attention(q, k, v).double()
+    small = torch.exp(-8 * k[0, 0, 0].double() * D**-0.5)  # a small key's weight, the dominating one's being 1
+    n = torch.arange(S, device=gpu, dtype=torch.float64)  # small keys that a query sees
+    total = n * small
+    want = (total / (1 + total))[:, None, None].expand_as(out)
+    half_unit, rounding = (2.0**-25 * n, 2.0**-11) if dtype == torch.float16 else (2.0**-8 * total, 2.0**-8)
+    bound = half_unit[:, None, None] + rounding * want + 2.0**-24
+    assert ((out - want).abs() <= bound).all(), ((out - want).abs() / bound).max().item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2e-2), (torch.float16, 1e-2)])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(12345, 4, 2, 128), (24000, 2, 1, 64)])
+def test_prefill_attention_of_long_prompts(gpu, dtype, tol, S, Hq, Hkv, D):
+    """The last 300 queries, which see every tile of a long prompt."""
+    print("case:", dict(S=S, Hq=Hq, Hkv=Hkv, D=D, dtype=str(dtype)), flush=True)
+    g = torch.Generator(device=gpu).manual_seed(S)
+    q, k, v = (torch.randn(S, h, D, generator=g, device=gpu).to(dtype) for h in (Hq, Hkv, Hkv))
+    out = rk.prefill_attention(q, k, v)[-300:].float()
+    mask = torch.arange(S, device=gpu) > torch.arange(S - 300, S, device=gpu)[:, None]
+    for h in range(Hq):
+        scores = q[-300:, h].float() @ k[:, h * Hkv // Hq].float().t().contiguous() * D**-0.5
+        want = scores.masked_fill_(mask, float("-inf")).softmax(-1) @ v[:, h * Hkv // Hq].float()
+        # outputs are sums of thousands of values of 1 / thousands each: hundredths, not ones
+        assert (out[:, h] - want).abs().max().item() <= tol * 0.1, h
+
+
 # ---- the prompt pass ------------------------------------------------------------------------
 
 
@@ -294,3 +341,92 @@ def test_prompt_pass_of_no_layers(prompt_device):
         row = model.model.embed_tokens.weight[TOKENS[-1]]
         want = torch.nn.functional.linear(rms_norm(row, model.model.norm.weight, 1e-6), model.lm_head.weight)
     assert torch.equal(model.prefill(TOKENS), want.float())
+
+
+def exact_prompt(model, tokens):
+    """Logits of the last token and each layer's keys and values, in float64
+    from the model's weights."""
+    cfg, n = model.config, len(tokens)
+    D, groups = cfg.head_dim, cfg.num_attention_heads // cfg.num_key_value_heads
+
+    def norm(x, m):
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + m.eps) * m.weight.double()
+
+    def linear(x, m):
+        y = x @ m.weight.double().t().contiguous()
+        return y if m.bias is None else y + m.bias.double()
+
+    x = model.model.embed_tokens.weight[tokens].double()
+    angle = torch.arange(n, device=x.device).double()[:, None] * cfg.rope_theta ** (
+        -torch.arange(0, D, 2, device=x.device).double() / D)
+    cos, sin = (torch.cat((f, f), -1)[:, None] for f in (angle.cos(), angle.sin()))
+    mask = torch.ones(n, n, dtype=torch.bool, device=x.device).triu(1)
+    kv = []
+    for layer in model.model.layers:
+        h, a = norm(x, layer.input_layernorm), layer.self_attn
+        q, k, v = (linear(h, p).view(n, -1, D) for p in (a.q_proj, a.k_proj, a.v_proj))
+        q, k = (t * cos + torch.cat((-t[..., D // 2:], t[..., : D // 2]), -1) * sin for t in (q, k))
+        kv += [k, v]
+        heads = []
+        for i in range(cfg.num_attention_heads):
+            scores = (q[:, i] @ k[:, i // groups].t().contiguous() * D**-0.5).masked_fill(mask, float("-inf"))
+            heads.append(scores.softmax(-1) @ v[:, i // groups])
+        x = x + linear(torch.cat(heads, -1), a.o_proj)
+        h = norm(x, layer.post_attention_layernorm)
+        x = x + linear(torch.nn.functional.silu(linear(h, layer.mlp.gate_proj)) * linear(h, layer.mlp.up_proj),
+                       layer.mlp.down_proj)
+    return [linear(norm(x[-1], model.model.norm), model.lm_head), *kv]
+
+
+class Written:
+    """A cache that keeps what is written to it."""
+
+    def __init__(self):
+        from types import SimpleNamespace
+
+        self.rows = []
+        self.storage = SimpleNamespace(requests={"r": SimpleNamespace(lengths=[0])})
+
+    def write(self, request_id, layer, k, v):
+        assert request_id == "r" and layer == len(self.rows) // 2
+        self.rows += [k.clone(), v.clone()]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n", [1, 70, 333])
+def test_prompt_pass_is_as_exact_as_the_general_one(prompt_device, monkeypatch, dtype, head_dim, n):
+    """Logits and the keys and values of every layer, of the fused prompt pass
+    and of the general expressions, against float64. Both round at the same
+    places of each layer, so their errors are the same but for single
+    roundings that fall the other way: a quarter more is allowed, where a
+    residual, a norm, a position or a row that is not the right one would
+    show as an error of the size of the result."""
+    from nano_hisparse import model as model_module
+
+    print("case:", dict(test="prompt-exact", device=str(prompt_device), dtype=str(dtype), D=head_dim, n=n), flush=True)
+    model = prompt_model(prompt_device, dtype, head_dim, layers=3)
+    tokens = [(7 * i * i + 3 * i) % 128 for i in range(n)]
+    with torch.inference_mode():
+        want = exact_prompt(model, tokens)
+    passes = []
+    fused_pass = model_module.Model._prefill_layers
+
+    def counted(self, *a):
+        passes.append(1)
+        return fused_pass(self, *a)
+
+    monkeypatch.setattr(model_module.Model, "_prefill_layers", counted)
+    results = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(model_module, "_plain_layer", lambda layer, dtype: False)
+        cache = Written()
+        logits = model.prefill(tokens, cache, "r")
+        assert torch.equal(logits, model.prefill(tokens))  # without a cache
+        results.append([logits, *cache.rows])
+    assert len(passes) == 2  # the fused pass ran, with and without the cache, and only in the first round
+    for name, exact, fused, general in zip(["logits", *"kvkvkv"], want, *results):
+        size = exact.norm()
+        a, b = ((r.double() - exact).norm() / size for r in (fused, general))
+        assert a <= 1.25 * b and b <= 3e-2, (name, a.item(), b.item())
