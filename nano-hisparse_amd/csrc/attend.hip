@@ -37,22 +37,6 @@ constexpr int kAttendThreads = 512;
 constexpr int kAttendWaves = kAttendThreads / kWave;
 constexpr int kMaxSplits = 32;
 constexpr int kMinRowsPerSplit = 32;  // the workspace holds partials for splits of this many rows
-// Fewest rows of a split, where fewer than one workgroup per CU leaves room
-// to split: a split costs the merge's store -> atomic -> load chain and every
-// further one lengthens the merge, while one workgroup reads several hundred
-// rows in a round trip or two. attend_kernel: four row groups of its eight
-// waves, at most kSplitRows. us at 32 rows per split / these, every launch on
-// rows untouched for 700 MB of other reads: one request of 4/2 heads of 64,
-// fp32: 128 rows 8.8 / 5.5, 512 rows 16.2 / 9.4, 2048 rows 25.5 / 13.0, and
-// eight of them 9.9 / 6.6, 13.1 / 9.8, 14.8 / 14.0; 14/2 heads of 64, bf16,
-// 2048 rows 35.2 / 16.2; 32/8 heads of 128, fp32: 512 rows 22.6 / 13.3 (four
-// requests 13.7 / 14.0, the most lost of 144 shapes), 2048 rows 24.2 / 18.7.
-// attend_mfma_kernel (128 rows per split / 256), 32/8 heads of 128, bf16: 256
-// rows 10.5 / 8.4, 2048 rows 12.5 / 11.2; 2 requests x 2048 rows 14.6 / 12.2,
-// 4 x 1024 12.8 / 11.8, 8 x 512 12.5 / 11.6, 8 x 256 11.2 / 8.8; 28/4 heads
-// of 128: 1 x 1024 13.6 / 13.9, 4 x 2048 18.0 / 15.1.
-constexpr int kSplitRows = 512;
-constexpr int kMSplitRows = 256;
 constexpr int kStage = 4096;  // row indices staged in LDS per pass (16 KiB)
 constexpr int kStagePerThread = kStage / kAttendThreads;
 constexpr int kIssueGroups = 2;  // row groups whose loads a wave issues together
@@ -1085,6 +1069,59 @@ static int max_splits_for(int n_rows) {
   return s < 1 ? 1 : s > kMaxSplits ? kMaxSplits : s;
 }
 
+// Splits of a row list for attend_mfma_kernel where compute units are left to
+// split for, of 256 rows: a split costs the merge's store -> atomic -> load
+// chain and every further one lengthens the merge, while a workgroup reads 256
+// rows in a round trip or two. Rounded up: one split more is cheaper than a
+// block of 128 rows more for each (28/4 heads of 128, bf16: 640 rows in 2 / 3
+// / 5 splits 16.2 / 13.6 / 13.9 us, 1024 in 3 / 4 / 8 16.6 / 13.9 / 13.6).
+// Two exceptions: with up to four (request, KV head) pairs, eight splits of
+// one block each (13.6 above); with half as many workgroups as CUs, lists of
+// three blocks stay whole (16 requests x 384 rows of 32/8 heads 12.3, two
+// splits 12.9). us at 128 rows per split / these, every launch on rows
+// untouched for 450 MB or more of other reads, 32/8 heads: 256 rows 10.5 /
+// 8.4, 2048 rows 12.5 / 11.2; 2 requests x 2048 rows 14.6 / 12.2, 4 x 1024
+// 12.8 / 11.8, 8 x 512 12.5 / 11.6.
+static int m_splits(int n_rows, int blocks, int kv_items) {
+  if (kv_items <= 4 && blocks == 8) return 8;
+  if (kv_items >= 128 && blocks <= 3) return 1;
+  return (n_rows + 255) / 256;
+}
+
+// Splits of a row list for attend_kernel, at most `most` (one workgroup per
+// CU), by the passes of its loop that the list takes (a pass: the rows whose
+// loads the eight waves issue together, 128 of 128 fp32 elements, 256 of 64,
+// 512 of 64 16-bit elements). A merge costs ~2.4 us for two splits and 0.5 to
+// 1.5 more for each further one, a pass ~1 to 4 us: so a pass per split up to
+// five or six, two per split beyond, at most eight splits or one per six
+// passes (a split's cost and a pass's balance as the root of their number; 8/2
+// heads of 256, fp32, 4096 rows in 64 passes: s8 32.4 us, s10 30.7, s16 28.7,
+// s32 34.6; 16/2 heads of 512, 2048 rows in 64: 57.0, 59.4, 69.5, 112.8), and no
+// more splits than give the same few row groups (half passes) to each. Lists of two
+// passes and a little more stay whole (of a pass and a half, where a pass is
+// 512 rows). us of splits s, every launch on rows untouched for 450 MB or more
+// of other reads: one request of 4/2 heads of 64, fp32: 512 rows s1 9.5, s2
+// 9.6; 1024 rows s1 14.1, s2 12.0, s4 10.8; 2048 rows s4 13.1, s8 13.2; 4096
+// rows s4 17.7, s8 15.6, s16 17.7. 32/8 heads of 128, fp32: 512 rows s1 15.4,
+// s2 13.4, s4 12.5; 1024 rows s4 15.0, s8 16.4; 4096 rows s4 29.2, s8 24.0,
+// s16 27.3. 14/2 heads of 64, bf16: 2048 rows s2 18.3, s4 16.0, s8 17.3. With
+// one head per workgroup the rows' loads bound it from 128 workgroups on: 16
+// requests of 8/8 heads of 128, fp32, 256 rows s1 11.9, s2 13.5; 640 rows
+// 21.3, 21.7.
+static int pass_splits(int n_rows, int pass, int most) {
+  const int passes = (n_rows + pass - 1) / pass, limit = std::max(8, passes / 6);
+  int splits;
+  if (n_rows <= (pass >= 512 ? pass + pass / 2 : 2 * pass + pass / 4))
+    splits = 1;
+  else if (pass >= 512)
+    splits = std::min(passes, limit);
+  else
+    splits = passes <= (pass > 128 ? 6 : 5) ? passes : std::min((passes + 1) / 2, limit);
+  splits = std::min(splits, most);
+  const int groups = (n_rows + pass / 2 - 1) / (pass / 2), each = (groups + splits - 1) / splits;
+  return each > 4 ? splits : (groups + each - 1) / each;
+}
+
 // Compute units of the current device (cached per device).
 static int device_cus() {
   static std::mutex mu;
@@ -1195,11 +1232,13 @@ extern "C" int nhs_attend_rows(const void* query, int32_t q_dtype, int64_t q_bat
     m.qscale = a.qscale;
     const int target = cus > 0 ? cus : 256;
     int splits = (target + kv_items / 2) / kv_items;
+    // one workgroup of a CU's LDS: a few more than the CUs would run after all others
+    if (splits > 3 && splits * kv_items > target) splits = target / kv_items;
     if (splits < 1) splits = 1;
     if (splits > max_splits_for(n_rows)) splits = max_splits_for(n_rows);
     if (splits > kMMaxSplits) splits = kMMaxSplits;
-    splits = std::min(splits, std::max(1, n_rows / kMSplitRows));
     const int block = kMTile * kMWaves;
+    splits = std::min(splits, m_splits(n_rows, (n_rows + block - 1) / block, kv_items));
     int per = (n_rows + splits - 1) / splits;
     per = (per + block - 1) / block * block;
     splits = (n_rows + per - 1) / per;
@@ -1239,8 +1278,8 @@ extern "C" int nhs_attend_rows(const void* query, int32_t q_dtype, int64_t q_bat
   int splits = cus > 0 ? (cus + units / 2) / units : 1;
   if (splits < 1) splits = 1;
   if (splits > max_splits_for(n_rows)) splits = max_splits_for(n_rows);
-  const int group_rows = kAttendWaves * (kWave >> a.lpr_log2) * (C == 1 ? 4 : 2);  // U rows per lane slot
-  splits = std::min(splits, std::max(1, n_rows / std::min(4 * group_rows, kSplitRows)));
+  const int pass = kAttendWaves * (kWave >> a.lpr_log2) * (C == 1 ? 4 : 2) * kIssueGroups;  // U rows per lane slot
+  splits = G == 1 && units >= 128 && n_rows <= 5 * pass ? 1 : pass_splits(n_rows, pass, splits);
   if ((int64_t)units * splits > 0x7fffffff) return fail(NHS_ERR_UNSUPPORTED, "nhs_attend_rows: grid too large");
   a.kv_items = kv_items;
   a.n_splits = splits;

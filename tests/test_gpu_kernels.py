@@ -695,6 +695,25 @@ def test_attend_rows_where_the_split_count_changes(gpu, dtype, Hq, Hkv, D, P, N)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,P,N", [
+    # attend_kernel, by passes of 256 (64 x fp32), 128 (128 x fp32), 512 (64 x 16 bits) or 32 (512 x fp32) rows
+    (torch.float32, 1, 4, 2, 64, 16, 577), (torch.float32, 5, 4, 2, 64, 16, 1537), (torch.float32, 16, 4, 2, 64, 16, 912),
+    (torch.float32, 5, 32, 8, 128, 16, 289), (torch.float32, 5, 32, 8, 128, 16, 528),
+    (torch.float32, 1, 16, 4, 128, 64, 2049), (torch.float32, 1, 4, 1, 128, 64, 7000),
+    (torch.float32, 16, 8, 8, 128, 16, 640), (torch.float32, 16, 8, 8, 128, 16, 641),
+    (torch.bfloat16, 16, 14, 2, 64, 16, 769), (torch.float16, 1, 8, 2, 64, 16, 4097),
+    (torch.float32, 1, 4, 1, 512, 4, 33), (torch.float32, 1, 4, 1, 512, 4, 73), (torch.float32, 1, 4, 1, 512, 4, 2500),
+    # attend_mfma_kernel: 257 to 1024 rows, four (request, KV head) pairs, half a CU's worth and more of them
+    (torch.bfloat16, 1, 32, 8, 128, 64, 257), (torch.bfloat16, 1, 28, 4, 128, 64, 640),
+    (torch.float16, 1, 16, 4, 128, 64, 896), (torch.float16, 1, 16, 4, 128, 64, 897),
+    (torch.bfloat16, 1, 28, 4, 128, 64, 1025), (torch.bfloat16, 16, 32, 8, 128, 64, 384),
+    (torch.bfloat16, 16, 32, 8, 128, 64, 385), (torch.bfloat16, 5, 28, 4, 128, 64, 3088),
+])
+def test_attend_rows_of_lists_that_the_splits_do_not_divide(gpu, dtype, B, Hq, Hkv, D, P, N):
+    test_attend_rows_matches_oracle(gpu, dtype, dtype, B, Hq, Hkv, D, P, N, False)
+
+
+@pytest.mark.gpu
 def test_attend_fp32_rounds_its_accumulators_once_per_row_group(gpu):
     """fp32 attention over 4096 rows a workgroup (16 requests of 32/8 heads of
     128: one split, 256 rows per lane slot in 64 groups) against float64. A
