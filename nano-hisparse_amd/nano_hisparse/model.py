@@ -487,7 +487,7 @@ class Model(nn.Module):
             for step in steps:
                 step.forget_capture_events()
             # what the graph reads outside its own memory lives as long as it does
-            entry = {"cache": cache, "read": _Held(self.modules()), "items": items, "buffers": buffers, "graph": graph,
+            entry = {"cache": cache, "read": _Held(_tree(self)), "items": items, "buffers": buffers, "graph": graph,
                      "logits": logits, "stream": side, "tables": tables,
                      "workspaces": [step.workspace for step in steps]}
             graphs[key] = entry
@@ -503,12 +503,19 @@ class Model(nn.Module):
         return entry["logits"].clone()
 
 
+def _tree(module):
+    """A module and every module below it."""
+    modules = [module]
+    for m in modules:
+        modules.extend(c for c in m._modules.values() if c is not None)
+    return modules
+
+
 class _Held:
     """The parameters and child modules that some modules hold at one time,
     to tell later whether they hold the same ones at the same addresses."""
 
     def __init__(self, modules):
-        modules = list(modules)
         self.dicts = [d for m in modules for d in (m._parameters, m._buffers, m._modules) if d]
         self.children = [c for m in modules for c in m._modules.values()]  # held: their identities stay their own
         self.state = self._now()

@@ -453,20 +453,20 @@ def test_replaced_parameters_and_modules_are_noticed():
     """What a captured graph and the fused projections read is compared by
     address and layout: a graph replayed on other parameters would read the
     old ones' freed memory."""
-    from nano_hisparse.model import _Held
+    from nano_hisparse.model import _Held, _tree
 
     model = Model(ModelConfig(num_hidden_layers=2)).eval()
     attn, mlp = model.model.layers[1].self_attn, model.model.layers[0].mlp
-    read, fused = _Held(model.modules()), model._fused_projections()
+    read, fused = _Held(_tree(model)), model._fused_projections()
     assert not read.unchanged()  # fusing made the projections views of the fused tensors
-    read = _Held(model.modules())
+    read = _Held(_tree(model))
     model.load_state_dict(model.state_dict())  # in place
     assert read.unchanged() and model._fused_projections() is fused
     model.lm_head.weight = torch.nn.Parameter(model.lm_head.weight.detach().clone())
     assert not read.unchanged() and model._fused_projections() is fused  # not one of the fused
 
     def changed(change, refuses=True):
-        read, fused = _Held(model.modules()), model._fused_projections()
+        read, fused = _Held(_tree(model)), model._fused_projections()
         assert read.unchanged()
         change()
         assert not read.unchanged()
