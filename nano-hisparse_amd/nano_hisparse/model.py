@@ -1,10 +1,12 @@
 """A small Qwen2-shaped decoder that drives the sparse decode path.
 
-Reference: nano_hisparse/model.py:19-221. Dense layers (projections, RoPE,
-RMSNorm, SwiGLU) are torch operations, the prefill's causal attention of a
-bf16/fp16 GPU model is the MFMA flash kernel (nhs_prefill_attention); each
+Reference: nano_hisparse/model.py:19-221. Projections and SwiGLU are torch
+operations; in the prompt pass of a bf16/fp16 GPU model RMSNorm (with the
+residual add), RoPE and the causal attention are kernels
+(nhs_add_rmsnorm, nhs_rope, nhs_prefill_attention), elsewhere torch too. Each
 decode step appends K/V through the cache, selects pages with Quest on the
-GPU and attends over the selected rows with the HIP kernels. The module tree
+GPU and attends over the selected rows with the HIP kernels; the batched one
+runs its dense layers on kernels as well. The module tree
 (names and construction order) is the reference's, which is HF Qwen2's, so
 state dicts load either way and a seeded random init draws the same weights.
 """
@@ -293,7 +295,7 @@ class Model(nn.Module):
         work. Returns fp32 logits [B, vocab]; row b equals decode(tokens[b],
         request_ids[b]) up to the order of the dense layers' reductions.
 
-        graph=True (one group) replays the step's launches from a HIP graph
+        graph=True replays the step's launches from a HIP graph
         captured at the first step of this batch composition (see
         _decode_batch_graph): the same kernels on the same buffers, with no
         per-launch host work."""
