@@ -57,3 +57,16 @@ def cpu_kernels():
     cpu_provider.install()
     yield
     cpu_provider.uninstall()
+
+
+@pytest.fixture(scope="session")
+def native_launchers():
+    """The native launchers' module, for tests that call it without a GPU
+    (built first if nothing is)."""
+    from nano_hisparse import _hip
+
+    if not os.path.exists(_hip.LIB_PATH):
+        import __graft_entry__
+
+        __graft_entry__.build()
+    return _hip.load_launch()

@@ -449,7 +449,7 @@ def test_graph_groups_with_and_without_kept_rope_tables(gpu, monkeypatch):
     assert tokens[0] == tokens[1]
 
 
-def test_replaced_parameters_and_modules_are_noticed():
+def test_replaced_parameters_and_modules_are_noticed(native_launchers):
     """What a captured graph and the fused projections read is compared by
     address and layout: a graph replayed on other parameters would read the
     old ones' freed memory."""

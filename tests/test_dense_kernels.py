@@ -215,7 +215,7 @@ def test_no_table_is_made_while_a_stream_is_captured(monkeypatch):
     assert model._rope_tables(20) is kept and model._rope_tables(21) is None
 
 
-def test_rope_tables_go_with_what_they_were_made_for():
+def test_rope_tables_go_with_what_they_were_made_for(native_launchers):
     """Tables of an earlier dtype are dropped when new ones are made,
     clear_decode_graphs() drops all of them, and a copy of the model carries
     none along."""

@@ -353,7 +353,8 @@ def test_tables_after_prompt_writes_hold_every_page(device, tokens):
 
 @pytest.mark.parametrize("argument,value", [
     (8, -1), (8, np.int64(-1)), (9, np.int32(-1)), (9, torch.tensor(16)), (10, np.int64(0)), (12, -3)])
-def test_page_append_launcher_takes_any_integer_and_leaves_refusals_to_the_library(argument, value):
+def test_page_append_launcher_takes_any_integer_and_leaves_refusals_to_the_library(
+        native_launchers, argument, value):
     """Calls that the library refuses on the host, before anything is
     launched: block, rows or host page outside the page (a status, as through
     ctypes), given as whole numbers of any type."""
@@ -361,7 +362,7 @@ def test_page_append_launcher_takes_any_integer_and_leaves_refusals_to_the_libra
 
     call = [4096, 4096, 64, _hip.NHS_F32, 64, 16, 4096, 8192, 0, 0, 1, 4096, 0, 4096, 4096, 4096, 0]
     call[argument] = value
-    assert _hip.load_launch().append_page(*call) == -1
+    assert native_launchers.append_page(*call) == -1
     call[argument] = "page"
     with pytest.raises(TypeError):
-        _hip.load_launch().append_page(*call)
+        native_launchers.append_page(*call)
