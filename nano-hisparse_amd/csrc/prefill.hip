@@ -135,7 +135,6 @@ __device__ __forceinline__ uint2 pf_read_tr(const char* p) {
 
 template <typename T, int D, int KSPLIT>
 __global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillArgs a) {
-  constexpr int kThreads = kPfThreads;
   constexpr int QW = kPfWaves / KSPLIT;  // waves of different queries
   constexpr int BM = 32 * QW;            // queries per workgroup
   constexpr int KS = D / 16;           // 16-wide k steps of Q.K
@@ -286,8 +285,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillAr
         for (int i = 0; i < 16; ++i) o[b][i] *= alpha;
     }
     const float ref = m == -INFINITY ? 0.f : m * a.scale_log2;
-    // weights rounded to the input dtype, packed as P^T B operands
+    // weights rounded to the input dtype, packed as P^T B operands; the
+    // denominator takes each tile's sum (in one chain over all tiles its error
+    // at 32768 keys is 6.6e-7 of it and not 3.1e-7)
     uint4 pb[4];
+    float tile_sum = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       uint32_t w[4];
@@ -296,10 +298,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_kernel(PrefillAr
         const float e0 = s[j >> 1][(j & 1) * 8 + 2 * x], e1 = s[j >> 1][(j & 1) * 8 + 2 * x + 1];
         w[x] = pf_pack<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(e0, a.scale_log2, -ref)),
                           __builtin_amdgcn_exp2f(__builtin_fmaf(e1, a.scale_log2, -ref)));
-        l = pf_add_pair<T>(w[x], l);
+        tile_sum = pf_add_pair<T>(w[x], tile_sum);
       }
       pb[j] = make_uint4(w[0], w[1], w[2], w[3]);
     }
+    l += tile_sum;
     // O^T += V^T P^T: dim block b, 16-key step j
 #pragma unroll
     for (int j = 0; j < 4; ++j)
