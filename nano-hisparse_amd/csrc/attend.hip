@@ -1096,10 +1096,10 @@ static int m_splits(int n_rows, int blocks, int kv_items) {
 // five or six, two per split beyond, at most eight splits or one per six
 // passes (a split's cost and a pass's balance as the root of their number; 8/2
 // heads of 256, fp32, 4096 rows in 64 passes: s8 32.4 us, s10 30.7, s16 28.7,
-// s32 34.6; 16/2 heads of 512, 2048 rows in 64: 57.0, 59.4, 69.5, 112.8), and no
-// more splits than give the same few row groups (half passes) to each. Lists of two
-// passes and a little more stay whole (of a pass and a half, where a pass is
-// 512 rows). us of splits s, every launch on rows untouched for 450 MB or more
+// s32 34.6; 16/2 heads of 512, 2048 rows in 64: 57.0, 59.4, 69.5, 112.8), and
+// no more splits than give the same few row groups (half passes) to each.
+// Lists of two passes and a little more stay whole (of a pass and a half,
+// where a pass is 512 rows). us of splits s, every launch on rows untouched for 450 MB or more
 // of other reads: one request of 4/2 heads of 64, fp32: 512 rows s1 9.5, s2
 // 9.6; 1024 rows s1 14.1, s2 12.0, s4 10.8; 2048 rows s4 13.1, s8 13.2; 4096
 // rows s4 17.7, s8 15.6, s16 17.7. 32/8 heads of 128, fp32: 512 rows s1 15.4,
@@ -1232,7 +1232,8 @@ extern "C" int nhs_attend_rows(const void* query, int32_t q_dtype, int64_t q_bat
     m.qscale = a.qscale;
     const int target = cus > 0 ? cus : 256;
     int splits = (target + kv_items / 2) / kv_items;
-    // one workgroup of a CU's LDS: a few more than the CUs would run after all others
+    // a few workgroups more than the CUs make the launch longer than fewer, longer splits: 5 requests x 3088 rows of
+    // 28/4 heads in 13 splits (260 workgroups) 26.1 us, in 9 19.5
     if (splits > 3 && splits * kv_items > target) splits = target / kv_items;
     if (splits < 1) splits = 1;
     if (splits > max_splits_for(n_rows)) splits = max_splits_for(n_rows);

@@ -19,6 +19,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <new>
 #include <stdexcept>
 #include <vector>
 
@@ -488,45 +489,53 @@ PyObject* append_page(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 
 // ---- parameters --------------------------------------------------------------------------------
 
+// Of a tensor its address, dtype, sizes and strides; of any other object, and of a tensor without them, its identity.
+void add_state(std::vector<int64_t>& state, PyObject* value) {
+  const size_t before = state.size();
+  if (PyObject_TypeCheck(value, reinterpret_cast<PyTypeObject*>(THPVariableClass))) {
+    try {
+      const Tensor& t = THPVariable_Unpack(value);
+      state.push_back((int64_t)(uintptr_t)t.const_data_ptr());
+      state.push_back((int64_t)t.scalar_type() << 32 | t.dim());
+      for (int64_t s : t.sizes()) state.push_back(s);
+      for (int64_t s : t.strides()) state.push_back(s);
+      return;
+    } catch (const std::bad_alloc&) {
+      throw;
+    } catch (const std::exception&) {  // a sparse or wrapped tensor
+      PyErr_Clear();
+      state.resize(before);
+    }
+  }
+  state.push_back((int64_t)(uintptr_t)value);
+}
+
 // The bytes that tell whether the dicts (of modules' parameters and child
-// modules) hold what they held: each dict's size, and of each value a tensor's
-// address, dtype, sizes and strides or, of any other object and of a tensor
-// without them, its identity. For checks made on every step.
+// modules) hold what they held: each dict's size and its values' states. For
+// checks made on every step.
 PyObject* held_state(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (nargs != 1 || !PyList_CheckExact(a[0])) {
     PyErr_SetString(PyExc_TypeError, "held_state takes a list of dicts");
     return nullptr;
   }
-  std::vector<int64_t> state;
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); ++i) {
-    PyObject* dict = PyList_GET_ITEM(a[0], i);
-    if (!PyDict_Check(dict)) {
-      PyErr_SetString(PyExc_TypeError, "held_state takes a list of dicts");
-      return nullptr;
-    }
-    state.push_back(PyDict_Size(dict));
-    PyObject *key, *value;
-    Py_ssize_t at = 0;
-    while (PyDict_Next(dict, &at, &key, &value)) {
-      if (!PyObject_TypeCheck(value, reinterpret_cast<PyTypeObject*>(THPVariableClass))) {
-        state.push_back((int64_t)(uintptr_t)value);
-        continue;
+  try {
+    std::vector<int64_t> state;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); ++i) {
+      PyObject* dict = PyList_GET_ITEM(a[0], i);
+      if (!PyDict_Check(dict)) {
+        PyErr_SetString(PyExc_TypeError, "held_state takes a list of dicts");
+        return nullptr;
       }
-      const size_t before = state.size();
-      try {
-        const Tensor& t = THPVariable_Unpack(value);
-        state.push_back((int64_t)(uintptr_t)t.const_data_ptr());
-        state.push_back((int64_t)t.scalar_type() << 32 | t.dim());
-        for (int64_t s : t.sizes()) state.push_back(s);
-        for (int64_t s : t.strides()) state.push_back(s);
-      } catch (const std::exception&) {
-        state.resize(before);
-        state.push_back((int64_t)(uintptr_t)value);
-      }
+      state.push_back(PyDict_Size(dict));
+      PyObject *key, *value;
+      Py_ssize_t at = 0;
+      while (PyDict_Next(dict, &at, &key, &value)) add_state(state, value);
     }
+    return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(state.data()),
+                                     (Py_ssize_t)(state.size() * sizeof(int64_t)));
+  } catch (const std::bad_alloc&) {
+    return PyErr_NoMemory();
   }
-  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(state.data()),
-                                   (Py_ssize_t)(state.size() * sizeof(int64_t)));
 }
 
 #define NHS_METHOD(name) \

@@ -560,3 +560,20 @@ def test_token_ids_are_checked_for_a_plain_embedding_only():
     model.model.embed_tokens = Wrapped(64, 128)
     with pytest.raises(RuntimeError, match="GPU cache"):  # past the check of the ids
         model.decode_batch([64], ["a"], cache, 2)
+
+
+def test_held_state_of_odd_values(native_launchers):
+    """Values without an address or strides count by identity, an added or a
+    removed entry by the dicts' sizes; what is no list of dicts is refused."""
+    state = native_launchers.held_state
+    dense, sparse = torch.eye(3), torch.eye(3).to_sparse()
+    held = {"a": dense, "b": sparse, "c": None, "d": torch.empty(0), "e": torch.empty(2, device="meta")}
+    before = state([held, {}])
+    assert state([dict(held), {}]) == before
+    for name, value in (("a", dense.t()), ("a", dense[:2]), ("a", dense.view(torch.int32)), ("a", dense.clone()),
+                        ("b", torch.eye(3).to_sparse()), ("c", dense), ("e", torch.empty(3, device="meta"))):
+        assert state([{**held, name: value}, {}]) != before, name
+    assert state([{**held, "f": None}, {}]) != before and state([held, {"f": None}]) != before
+    for wrong in ((held,), [held, 1], 5):
+        with pytest.raises(TypeError):
+            state(wrong)
