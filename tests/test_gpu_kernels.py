@@ -682,11 +682,11 @@ def test_append_rows_at_the_edges_of_passes_and_chunks(gpu, dtype, P, Hkv, D):
 
 
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,P,N", [
-    # attend_kernel: one split up to two times its smallest size, then two and more (512 rows at 64 x fp32, 256 at 128 x fp32)
+    # attend_kernel: one split up to 576 rows of 64 x fp32, 288 of 128 x fp32, 768 of 64 x 16 bits; one per pass beyond
     (torch.float32, 4, 2, 64, 16, 512), (torch.float32, 4, 2, 64, 16, 1023), (torch.float32, 4, 2, 64, 16, 1024),
     (torch.float32, 4, 2, 64, 16, 1600), (torch.float32, 8, 2, 128, 64, 511), (torch.float32, 8, 2, 128, 64, 513),
     (torch.bfloat16, 14, 2, 64, 16, 1024), (torch.float32, 3, 3, 256, 8, 300),
-    # attend_mfma_kernel: splits of at least 256 rows
+    # attend_mfma_kernel: one split up to 256 rows, then one per 256
     (torch.bfloat16, 32, 8, 128, 64, 255), (torch.bfloat16, 32, 8, 128, 64, 511), (torch.float16, 32, 8, 128, 64, 512),
     (torch.bfloat16, 28, 4, 128, 32, 1025),
 ])
